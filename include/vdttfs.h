@@ -344,7 +344,10 @@ int vdttfs_net_set_windows(vdttfs_net* net, const int32_t* windows, int n_layers
  * (> 25 taps) take the generic integrator (path BINS, gather and ppw 0).
  * Pool and vmem layers have no plan.  set_plan(NULL) restores the built-in
  * choice; an unsupported request fails with VDTTFS_E_UNSUPPORTED and leaves
- * the layer's plan unchanged.  get_plan returns the resolved plan the next
+ * the layer's plan unchanged.  Where no field is asked for, a layer whose fire
+ * start is a quarter of its window or more may run on the split kernels (bin 0
+ * on the matrix cores), which have no plan fields: get_plan then names the plan
+ * that its counting forwards, and forwards with a pool fused into it, take.  get_plan returns the resolved plan the next
  * forward uses. */
 #define VDTTFS_PATH_AUTO   0
 #define VDTTFS_PATH_BINS   1

@@ -104,12 +104,24 @@ int ensure_merge_scratch(vdttfs_ctx* ctx, size_t list_elems, size_t bstart_elems
         if (ctx->mrg_list) VD_HIP(hipFree(ctx->mrg_list));
         if (ctx->mrg_bstart) VD_HIP(hipFree(ctx->mrg_bstart));
         ctx->mrg_list = ctx->mrg_bstart = nullptr;
+        ctx->mrg_list_elems = ctx->mrg_bstart_elems = 0;
         VD_TRY(grow(&ctx->mrg_list, &h1, e * sizeof(int2)));
         VD_TRY(grow(&ctx->mrg_bstart, &h2, b * 4));
         ctx->mrg_list_elems = e;
         ctx->mrg_bstart_elems = b;
     }
     return VDTTFS_OK;
+}
+
+bool ensure_split_scratch(vdttfs_ctx* ctx, size_t list_elems) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (ensure_merge_scratch(ctx, list_elems, 1) == VDTTFS_OK) return true;
+    (void)hipGetLastError();
+    return false;
 }
 
 static int check_consts(const vdttfs_consts* c) {
@@ -355,6 +367,14 @@ static int engine_layer(vdttfs_ctx* ctx, float* d_out, const float* d_in, const 
     const int64_t cap = merged_list_cap(s);
     const bool dense = plan_from_dense(ctx, s, p, counters != nullptr);
     const bool lds_list = plan_lds_list(ctx, s, p, counters != nullptr, false);
+    if (p.split && !counters) {
+        // as much as the named plan would take, so that a counting call of the
+        // layer finds its lists' scratch
+        const size_t need = split_scratch_bytes(s) / sizeof(int2) + 1, named = lds_list ? 0 : (size_t)(n_pix * cap);
+        if (ensure_split_scratch(ctx, need > named ? need : named))
+            return launch_integrate_split(ctx, d_out, d_in, d_lut_decay, ctx->mrg_list, d_kernel, d_bias, d_lut_th,
+                                          t_min, s);
+    }
     if (!lds_list)
         VD_TRY(ensure_merge_scratch(ctx, (size_t)(n_pix * cap), (size_t)n_pix * (ctx->c.T + 1)));
     if (dense)  // conv: merged lists straight from the dense map

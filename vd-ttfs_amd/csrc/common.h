@@ -76,6 +76,11 @@ int check_ctx(vdttfs_ctx* ctx);
 int ensure_ref_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols);
 int ensure_bin_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols);
 int ensure_merge_scratch(vdttfs_ctx* ctx, size_t list_elems, size_t bstart_elems);
+// The split integrator's scratch, in the merged lists' buffer: at least
+// list_elems entries of it.  false where it cannot be had (no memory, or the
+// stream is under capture, whose replays must not depend on a buffer that a
+// later call may replace): the caller then takes the layer's other kernels.
+bool ensure_split_scratch(vdttfs_ctx* ctx, size_t list_elems);
 
 // ---- kernel launchers (stream-ordered on ctx->stream) ----
 int launch_encode_log(vdttfs_ctx* ctx, const float* img, float* out, int64_t n, float tc, float td);
@@ -114,8 +119,12 @@ int merged_list_cap(const IntegShape& s);
 // the fused k_stream_dense), the weight gather (1: one c_out per lane, 2: two
 // events per dwordx4 load, 4: four c_out per lane) and output pixels per
 // wave.  Values as VDTTFS_PATH_* / vdttfs_layer_plan.
+// split (set by resolve_plan where the choice is the built-in one): forwards
+// without counters, with a LUT neuron and no fused pool take the split
+// integrator (k_split.hip) in place of the named kernels.
 struct LaunchPlan {
     int path = 0, gather = 0, ppw = 0;
+    bool split = false;
 };
 constexpr int kMaxPixPerWave = 8;
 // The plan's lists come from the bin-layout bucketize (the bins and window paths).
@@ -170,6 +179,14 @@ int launch_integrate_dense(vdttfs_ctx* ctx, float* out, const float* in, const f
                            const float* theta, int t_min, const IntegShape& s,
                            unsigned long long* counters, const CulifNeuron* culif = nullptr,
                            const LaunchPlan* plan = nullptr, const PoolIn* pool = nullptr);
+
+// The split integrator (k_split.hip): bin 0 on the matrix cores, the later
+// bins from per-column lists.  split_ok: the layers it can and should take;
+// split_scratch_bytes: the device scratch of one call.
+bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s);
+size_t split_scratch_bytes(const IntegShape& s);
+int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
+                           const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s);
 
 int launch_pool_min(vdttfs_ctx* ctx, const float* in, float* out, int B, int H_in, int W_in, int C);
 int launch_fc_vmem(vdttfs_ctx* ctx, const float* in, float* out, const float* W, const float* bias,

@@ -3984,7 +3984,8 @@ int plan_error(const IntegShape& sh, const char* what) {
 
 }  // namespace
 
-int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan& req, LaunchPlan* out) {
+namespace {
+int resolve_named(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan& req, LaunchPlan* out) {
     if (req.path < 0 || req.path > VDTTFS_PATH_WINDOW || req.gather < 0 || req.ppw < 0 || req.ppw > 64)
         return set_error(VDTTFS_E_INVALID, "plan: path %d, gather %d, ppw %d out of range", req.path,
                          req.gather, req.ppw);
@@ -4126,6 +4127,14 @@ int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan& 
         }
     }
     *out = p;
+    return VDTTFS_OK;
+}
+
+}  // namespace
+
+int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan& req, LaunchPlan* out) {
+    VD_TRY(resolve_named(ctx, sh, req, out));
+    out->split = !req.path && !req.gather && !req.ppw && split_ok(ctx, sh);
     return VDTTFS_OK;
 }
 
