@@ -239,7 +239,7 @@ struct MaskArgs {
 };
 
 constexpr int kMaskUnitsPerWave = 8;
-constexpr int kMaskPixPerWave = 16;  // consecutive output pixels per wave
+constexpr int kMaskPixPerWave = 16;  // most consecutive output pixels per wave
 constexpr int kMaskMaxCin = 3;  // taps held in registers and in 32-bit step masks: C_in * 9 <= 27
 
 __global__ __launch_bounds__(256) void k_culif_event_masks(MaskArgs a) {
@@ -271,139 +271,218 @@ __global__ __launch_bounds__(256) void k_culif_event_masks(MaskArgs a) {
     }
 }
 
-// One wave per kMaskPixPerWave consecutive output pixels and a 64-wide c_out
-// block (lanes = c_out), four waves of one c_out block per workgroup; NK =
-// C_in * 9 taps, the lane's NK weights in registers.  Per 64-step block the
-// tap masks are transposed so that lane t holds the taps with input at step t
-// (NK <= 32 bits); a step with input then visits only its set taps, in
-// ascending k, one add each (fma(w, 1, in) is exactly in + w).  All T steps
-// run the neuron update (a step without input still decays I and adds it to
-// V).  The wave's live neurons are an SGPR lane mask and each lane counts the
-// steps it has lived through, which is its spike step once it fires; steps
-// are tested eight at a time against one byte of the block's input mask.
+// One wave per `ppw` consecutive output pixels and a 64-wide c_out block (lanes
+// = c_out), four waves of one c_out block per workgroup; NK = C_in * 9 taps.
+// The input currents of 32 steps are a dense product on the matrix cores:
+// v_mfma_f32_32x32x2 takes steps as rows, c_out as columns (two tiles) and taps
+// as k, two a step, as two fmas in k order, so a step's chain is the
+// reference's, and a tap without input adds fma(w, 0, in) = in (finite
+// weights).  A's elements come from the tap masks, two scalar words picking
+// 1.0 or 0 per lane; a pair of taps without input in the 32 steps is skipped,
+// and 32 steps without input in any tap need no product.  16 permlane swaps
+// then leave lane c with all 32 steps of c_out c, and the neuron steps run
+// straight-line: four vector instructions a step.  The wave's live neurons are
+// an SGPR lane mask and each lane counts the steps it has lived through, which
+// is its spike step once it fires.
+//
+// Bound by the matrix unit (128 cycles per pair of taps and 32 steps) and the
+// neuron steps.  Visiting the set taps one by one (a scalar bit scan and an
+// indexed register add each) took 1,370 us on CuLIF-7's conv1 (B=64, 128x128,
+// 2 -> 64, T=64) where this takes 849.
 template <int NK>
-__global__ __launch_bounds__(256) void k_culif_conv1_mask(RawArgs a, const uint64_t* __restrict__ mask,
-                                                          const uint32_t* __restrict__ nonbin, int nblk) {
-    static_assert(NK <= 32, "tap masks are 32-bit");
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_culif_conv1_mask(
+    RawArgs a, const uint64_t* __restrict__ mask, const uint32_t* __restrict__ nonbin, int nblk, int ppw) {
+    static_assert(NK <= 32, "tap flags are 32-bit");
+    typedef float f16v __attribute__((ext_vector_type(16)));
+    constexpr int NP = (NK + 1) / 2;  // pairs of taps
     const int wave = uniform(threadIdx.x >> 6);
     const int64_t b = blockIdx.x;
     const int cb = (int)(b % a.n_cblk);
     const int lane = lane_id();
+    const int h = lane >> 5, l = lane & 31;
     const int c = cb * 64 + lane;
     const bool ok = c < a.C_out;
-    float w[NK];
+    float w[NP][2];  // B: tap 2s + h, c_out l of each tile
 #pragma unroll
-    for (int k = 0; k < NK; ++k) w[k] = ok ? a.W[(int64_t)c * NK + k] : 0.0f;
+    for (int s = 0; s < NP; ++s)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const int k = 2 * s + h, co = cb * 64 + 32 * v + l;
+            w[s][v] = (k < NK && co < a.C_out) ? a.W[(int64_t)co * NK + k] : 0.0f;
+        }
     // lane k < NK: tap k = (ci, ky, kx) in the reference's order, as a site
     // offset from (n, ci = 0, y, x)
     const int tk = lane < NK ? lane : 0;
     const int tdy = (tk % 9) / 3 - 1, tdx = tk % 3 - 1;
     const int64_t toff = ((int64_t)(tk / 9) * a.H + tdy) * a.Wd + tdx;
-    const int pix0 = uniform((int)((b / a.n_cblk) * 4 + wave)) * kMaskPixPerWave;  // < 2^31 (host check)
-    for (int pq = 0; pq < kMaskPixPerWave; ++pq) {
-        const int pix = pix0 + pq;
-        if (pix >= a.n_pix) return;  // uniform per wave
-        const int x = pix % a.Wd;
-        const int y = (pix / a.Wd) % a.H;
-        const int n = pix / (a.Wd * a.H);
-        // this lane's tap site, or none out of bounds (skipped, as the
-        // reference does)
+    const int pix0 = uniform((int)((b / a.n_cblk) * 4 + wave)) * ppw;  // < 2^31 (host check)
+    // A pixel's tap masks: lane k's tap site (none out of bounds: skipped, as
+    // the reference does), its mask of the first 64 steps with input, and
+    // whether a nonzero input there is not 1.0.  The next pixel's are loaded
+    // while one is integrated.
+    struct Taps {
+        int64_t site;
+        bool in, nb;
+        uint64_t mk;
+    };
+    auto fetch = [&](int n, int y, int x) -> Taps {
+        Taps p;
         const int iy = y + tdy, ix = x + tdx;
-        const bool tap_in = lane < NK && iy >= 0 && iy < a.H && ix >= 0 && ix < a.Wd;
-        const int64_t site = ((int64_t)n * a.C_in * a.H + y) * a.Wd + x + toff;
-        auto tap_site = [&](int k) -> int64_t {  // wave-uniform, for a tap with input
-            const uint64_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)site, k);
-            const uint64_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)site >> 32), k);
-            return (int64_t)(lo | (hi << 32));
-        };
+        p.in = lane < NK && iy >= 0 && iy < a.H && ix >= 0 && ix < a.Wd;
+        p.site = ((int64_t)n * a.C_in * a.H + y) * a.Wd + x + toff;
+        p.mk = 0;
+        p.nb = false;
+        if (p.in) {
+            p.mk = mask[p.site * nblk];
+            p.nb = nonbin[p.site * nblk] != 0;
+        }
+        return p;
+    };
+    if (pix0 >= a.n_pix) return;  // uniform per wave
+    const int pix1 = pix0 + ppw < a.n_pix ? pix0 + ppw : (int)a.n_pix;
+    int x = pix0 % a.Wd, y = (pix0 / a.Wd) % a.H, n = pix0 / (a.Wd * a.H);
+    Taps nxt = fetch(n, y, x);
+    for (int pix = pix0; pix < pix1; ++pix) {
+        const Taps cur = nxt;
+        const int cx = x, cy = y, cn = n;
+        if (++x == a.Wd) {
+            x = 0;
+            if (++y == a.H) {
+                y = 0;
+                ++n;
+            }
+        }
+        if (pix + 1 < pix1) nxt = fetch(n, y, x);
+        const int64_t site = cur.site;
         float I = 0.0f, V = 0.0f;
         int lived = 0;  // steps survived: the spike step once the lane fired
         const uint64_t all = __ballot(ok);
         uint64_t alive = all;
+        auto neuron = [&](float in) __attribute__((always_inline)) {
+            I = __builtin_fmaf(I, a.decay, in);
+            V = V + I;
+            alive &= ~__builtin_amdgcn_ballot_w64(V >= a.th);
+            lived = add_lane_bit(lived, alive);
+        };
+        // eight steps: where no live neuron reaches the threshold in them, all
+        // live through all eight
+        auto neuron8 = [&](const float (&in)[8]) __attribute__((always_inline)) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                I = __builtin_fmaf(I, a.decay, in[u]);
+                V = V + I;
+                v[u] = V;
+            }
+            float top = v[0];  // fmaxf leaves a NaN out, which reaches no threshold
+#pragma unroll
+            for (int u = 1; u < 8; ++u) top = fmaxf(top, v[u]);
+            if ((__builtin_amdgcn_ballot_w64(top >= a.th) & alive) == 0) {  // uniform
+                lived += __builtin_amdgcn_inverse_ballot_w64(alive) ? 8 : 0;
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    alive &= ~__builtin_amdgcn_ballot_w64(v[u] >= a.th);
+                    lived = add_lane_bit(lived, alive);
+                }
+            }
+        };
         for (int tb = 0; tb < nblk && alive; ++tb) {
-            // lane k's tap: its mask of steps with input, and whether a
-            // nonzero input is not 1.0
-            uint64_t mk = 0;
-            bool nbk = false;
-            if (tap_in) {
-                mk = mask[site * nblk + tb];
-                nbk = nonbin[site * nblk + tb] != 0;
+            uint64_t mk = cur.mk;
+            bool nbk = cur.nb;
+            if (tb > 0) {
+                mk = 0;
+                nbk = false;
+                if (cur.in) {
+                    mk = mask[site * nblk + tb];
+                    nbk = nonbin[site * nblk + tb] != 0;
+                }
             }
             const uint32_t nbm = (uint32_t)__ballot(nbk);  // bit k: tap k (NK <= 32)
-            uint32_t tapm = 0;  // lane t: taps with input at step t0 + t
-            if (__ballot(mk != 0)) {  // the transpose, for a block with any input
-                const int mlo = (int)(uint32_t)mk, mhi = (int)(uint32_t)(mk >> 32);
-#pragma unroll
-                for (int k = 0; k < NK; ++k) {
-                    const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(mlo, k) |
-                                       ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(mhi, k) << 32);
-                    tapm |= (__builtin_amdgcn_inverse_ballot_w64(m) ? 1u : 0u) << k;
-                }
-            }
-            const uint64_t any = __ballot(tapm != 0);  // steps with input (none at t >= T)
-            const int t0 = tb * 64;
-            const int tn = (a.T - t0) < 64 ? (a.T - t0) : 64;
-            // the input current of step t0 + t, which has input in some tap
-            // (so tm != 0); NB: some tap's values are not all 1.0
-            auto input = [&](int t, auto nb) -> float {
-                uint32_t tm = (uint32_t)__builtin_amdgcn_readlane((int)tapm, t);
-                float in = 0.0f;
-                if (decltype(nb)::value && (tm & nbm)) {
-                    // an input value other than 1.0 at this step (rare)
-                    do {
-                        const int k = __builtin_ctz(tm);
-                        tm &= tm - 1;
-                        const float v = ((nbm >> k) & 1) ? a.data[(int64_t)tap_site(k) * a.T + t0 + t] : 1.0f;
-                        in = __builtin_fmaf(w[k], v, in);
-                    } while (tm);
-                } else {
-                    do {
-                        const int k = __builtin_ctz(tm);
-                        tm &= tm - 1;
-                        in = in + w[k];
-                    } while (tm);
-                }
-                return in;
-            };
-            auto neuron = [&](float in) {
-                I = __builtin_fmaf(I, a.decay, in);
-                V = V + I;
-                alive &= ~__builtin_amdgcn_ballot_w64(V >= a.th);
-                lived = add_lane_bit(lived, alive);
-            };
-            auto run = [&](auto nb) {
-                // whole groups of 8 steps, then the last, partial group of T
-                int t8 = 0;
-                int first = t0 == 0 ? 1 : 0;  // the group holding step 0 never skips
-                for (; t8 + 8 <= tn; t8 += 8) {
-                    const uint32_t a8 = (uint32_t)(any >> t8) & 0xffu;
-                    // steps without input while every lane's current is zero
-                    // change nothing: I stays 0, V stays V (the threshold is
-                    // fixed), and a lane with V >= th would have fired at the
-                    // step before (none precedes step 0); its live lanes live
-                    // through them
-                    const int key = (int)a8 | first;
-                    first = 0;
-                    if (key == 0) {
+            const bool silent = __ballot(mk != 0) == 0;
+            for (int half = 0; half < 2 && alive; ++half) {
+                const int t0 = tb * 64 + 32 * half;
+                if (t0 >= a.T) break;
+                const int mh = half ? (int)(uint32_t)(mk >> 32) : (int)(uint32_t)mk;
+                if (silent || __ballot(mh != 0) == 0) {
+                    // Steps without input: while every lane's current is zero
+                    // they change nothing (I stays 0, V stays, the threshold is
+                    // fixed, and a lane with V >= th would have fired at the
+                    // step before; none precedes step 0), and the live lanes
+                    // live through them.
+                    int left = a.T - t0 < (silent ? 64 : 32) ? a.T - t0 : (silent ? 64 : 32);
+                    if (t0 == 0) {
+                        neuron(0.0f);
+                        --left;
+                    }
+                    while (left > 0 && alive) {
                         if (__builtin_amdgcn_ballot_w64(I != 0.0f) == 0) {
-                            lived += __builtin_amdgcn_inverse_ballot_w64(alive) ? 8 : 0;
-                            continue;
+                            lived += __builtin_amdgcn_inverse_ballot_w64(alive) ? left : 0;
+                            break;
+                        }
+                        if (left >= 8) {
+                            const float zero[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                            neuron8(zero);
+                            left -= 8;
+                        } else {
+                            neuron(0.0f);
+                            --left;
                         }
                     }
+                    if (silent) break;  // both halves
+                    continue;
+                }
+                const int tn = a.T - t0 < 32 ? a.T - t0 : 32;
+                f16v acc0, acc1;
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) neuron((a8 & (1u << u)) ? input(t8 + u, nb) : 0.0f);
-                    if (alive == 0) return;
+                for (int r = 0; r < 16; ++r) acc0[r] = acc1[r] = 0.0f;
+                auto product = [&](auto nb) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int s = 0; s < NP; ++s) {
+                        const uint32_t m0 = (uint32_t)__builtin_amdgcn_readlane(mh, 2 * s);
+                        const uint32_t m1 = 2 * s + 1 < NK ? (uint32_t)__builtin_amdgcn_readlane(mh, 2 * s + 1) : 0;
+                        const uint64_t m = (uint64_t)m0 | ((uint64_t)m1 << 32);
+                        if (m != 0) {  // uniform
+                            const bool on = __builtin_amdgcn_inverse_ballot_w64(m);
+                            float v = on ? 1.0f : 0.0f;
+                            if (decltype(nb)::value && ((nbm >> (2 * s)) & 3u)) {  // an input value other than 1.0 (rare): row l's value itself
+                                const int k = 2 * s + h;
+                                const int64_t sk = __shfl(site, k, 64);
+                                if (on) v = a.data[sk * a.T + t0 + l];
+                            }
+                            acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v, w[s][0], acc0, 0, 0, 0);
+                            acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v, w[s][1], acc1, 0, 0, 0);
+                        }
+                    }
+                };
+                if (nbm)
+                    product(std::true_type{});
+                else
+                    product(std::false_type{});
+                // lane (h, l) holds steps 8 (r / 4) + 4 h + r % 4 of c_out l and
+                // 32 + l: the swap gives every lane its own c_out's steps
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    float in[8];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc0[4 * r4 + r]),
+                                                                        __float_as_uint(acc1[4 * r4 + r]), false, false);
+                        in[r] = __uint_as_float(p[0]);
+                        in[4 + r] = __uint_as_float(p[1]);
+                    }
+                    if (8 * r4 + 8 <= tn) {
+                        neuron8(in);
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            if (8 * r4 + u < tn) neuron(in[u]);
+                    }
                 }
-                if (t8 < tn) {
-                    const uint32_t a8 = (uint32_t)(any >> t8) & 0xffu;
-                    for (int u = 0; u < tn - t8; ++u) neuron((a8 & (1u << u)) ? input(t8 + u, nb) : 0.0f);
-                }
-            };
-            if (nbm) run(std::true_type{});
-            else run(std::false_type{});
+            }
         }
         if (ok)
-            a.out[(int64_t)n * a.sN + (int64_t)c * a.sC + (int64_t)y * a.sY + (int64_t)x * a.sX] =
+            a.out[(int64_t)cn * a.sN + (int64_t)c * a.sC + (int64_t)cy * a.sY + (int64_t)cx * a.sX] =
                 __builtin_amdgcn_inverse_ballot_w64(alive) ? kInfTime : (float)lived;
         if (a.fired && lane == 0) a.fired[pix] = (all & ~alive) != 0 ? 1 : 0;
     }
@@ -1045,20 +1124,25 @@ int launch_culif_conv1_mask(vdttfs_ctx* ctx, const float* data, float* out, cons
     if (mblocks > 0x7fffffff) return set_error(VDTTFS_E_UNSUPPORTED, "culif_conv1_mask: grid too large");
     hipLaunchKernelGGL(k_culif_event_masks, dim3((unsigned)mblocks), dim3(256), 0, ctx->stream, m);
     VD_HIP(hipGetLastError());
-    const int64_t blocks = ((a.n_pix + 4 * kMaskPixPerWave - 1) / (4 * kMaskPixPerWave)) * a.n_cblk;
+    // pixels per wave: 16 amortise a wave's weights where that leaves eight
+    // waves per SIMD, fewer on smaller maps (33 samples of 32x32, T=160: 422 ->
+    // 98 us)
+    int ppw = (int)(a.n_pix * a.n_cblk / 8192);
+    ppw = ppw < 1 ? 1 : (ppw > kMaskPixPerWave ? kMaskPixPerWave : ppw);
+    const int64_t blocks = ((a.n_pix + 4 * ppw - 1) / (4 * ppw)) * a.n_cblk;
     if (blocks > 0x7fffffff) return set_error(VDTTFS_E_UNSUPPORTED, "culif_conv1_mask: grid too large");
     switch (C_in) {
         case 1:
             hipLaunchKernelGGL(k_culif_conv1_mask<9>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a,
-                               mask, nonbin, nblk);
+                               mask, nonbin, nblk, ppw);
             break;
         case 2:
             hipLaunchKernelGGL(k_culif_conv1_mask<18>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a,
-                               mask, nonbin, nblk);
+                               mask, nonbin, nblk, ppw);
             break;
         default:
             hipLaunchKernelGGL(k_culif_conv1_mask<27>, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a,
-                               mask, nonbin, nblk);
+                               mask, nonbin, nblk, ppw);
             break;
     }
     VD_HIP(hipGetLastError());
