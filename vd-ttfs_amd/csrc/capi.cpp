@@ -372,8 +372,11 @@ static int engine_layer(vdttfs_ctx* ctx, float* d_out, const float* d_in, const 
         // layer finds its lists' scratch
         const size_t need = split_scratch_bytes(s) / sizeof(int2) + 1, named = lds_list ? 0 : (size_t)(n_pix * cap);
         if (ensure_split_scratch(ctx, need > named ? need : named))
-            return launch_integrate_split(ctx, d_out, d_in, d_lut_decay, ctx->mrg_list, d_kernel, d_bias, d_lut_th,
-                                          t_min, s);
+            return p.split == kSplitLists
+                       ? launch_integrate_lists(ctx, d_out, d_in, d_lut_decay, ctx->mrg_list, d_kernel, d_bias,
+                                                d_lut_th, t_min, s, nullptr)
+                       : launch_integrate_split(ctx, d_out, d_in, d_lut_decay, ctx->mrg_list, d_kernel, d_bias,
+                                                d_lut_th, t_min, s);
     }
     if (!lds_list)
         VD_TRY(ensure_merge_scratch(ctx, (size_t)(n_pix * cap), (size_t)n_pix * (ctx->c.T + 1)));

@@ -121,11 +121,13 @@ int merged_list_cap(const IntegShape& s);
 // wave.  Values as VDTTFS_PATH_* / vdttfs_layer_plan.
 // split (set by resolve_plan where the choice is the built-in one): forwards
 // without counters, with a LUT neuron and no fused pool take the split
-// integrator (k_split.hip) in place of the named kernels.
+// integrator (1) or the column lists (2; k_split.hip) in place of the named
+// kernels.
 struct LaunchPlan {
     int path = 0, gather = 0, ppw = 0;
-    bool split = false;
+    int split = 0;
 };
+constexpr int kSplitDense = 1, kSplitLists = 2;
 constexpr int kMaxPixPerWave = 8;
 // The plan's lists come from the bin-layout bucketize (the bins and window paths).
 inline bool plan_bins(const LaunchPlan& p) { return p.path == VDTTFS_PATH_BINS || p.path == VDTTFS_PATH_WINDOW; }
@@ -187,6 +189,13 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s);
 size_t split_scratch_bytes(const IntegShape& s);
 int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
                            const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s);
+
+// The same lists over every bin, with the LUT or the CuLIF neuron (windows past
+// 64 steps); in split_scratch_bytes of scratch.
+bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s);
+int launch_integrate_lists(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
+                           const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s,
+                           const CulifNeuron* culif);
 
 int launch_pool_min(vdttfs_ctx* ctx, const float* in, float* out, int B, int H_in, int W_in, int C);
 int launch_fc_vmem(vdttfs_ctx* ctx, const float* in, float* out, const float* W, const float* bias,

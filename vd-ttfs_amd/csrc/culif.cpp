@@ -203,6 +203,8 @@ int create_impl(vdttfs_culif_net* net, const vdttfs_culif_layer* layers, int n) 
                 if (cols * d.C_in > max_ev) max_ev = cols * d.C_in;
                 if (cols > max_cols) max_cols = cols;
                 if (n_pix * l.list_cap > max_list) max_list = n_pix * l.list_cap;
+                const int64_t split_list = (int64_t)(split_scratch_bytes(sh) / sizeof(int2)) + 1;
+                if (split_list > max_list) max_list = split_list;
                 if (n_pix * (T + 1) > max_bstart) max_bstart = n_pix * (T + 1);
                 break;
             }
@@ -314,6 +316,11 @@ int forward_impl(vdttfs_culif_net* net, const float* d_data, int32_t* d_pred, ui
                 // map (the bin-layout bucketize then only counts retained events)
                 LaunchPlan plan;
                 VD_TRY(resolve_plan(ctx, sh, LaunchPlan{}, &plan));
+                if (!count_here && lists_ok(ctx, sh)) {
+                    VD_TRY(launch_integrate_lists(ctx, l.out, cur, net->ones, net->list, l.W, nullptr, nullptr, 0, sh,
+                                                  &nrn));
+                    break;
+                }
                 const bool dense = plan_from_dense(ctx, sh, plan, count_here);
                 if (!dense || count_here)
                     VD_TRY(launch_bucketize_bins(ctx, cur, cols, d.C_in, net->ones, net->ev, net->off,

@@ -31,7 +31,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
-constexpr int kSplitMaxT = 128;   // two blocks of 64 bins
+constexpr int kSplitMaxT = 256;   // four blocks of 64 bins
 constexpr int kSplitMaxTaps = 25;
 constexpr int kLatePad = 32;      // zeroed entries after the list (k_late reads up to four quads ahead)
 constexpr int kLateMaxWaves = 4;
@@ -51,7 +51,7 @@ struct LateThr {
 
 struct SplitArgs {
     const float* in;     // [cols][C_in] spike times
-    float* a0;           // [cols][Cp] bin-0 factors, C_in padded with zeros to whole groups of 4 HL; element
+    float* a0;           // null: no bin-0 factors, and the lists hold bin 0's events too; else [cols][Cp] bin-0 factors, C_in padded with zeros to whole groups of 4 HL; element
                          // HL s + h of a group at 4 h + s (k_gemm0's lane h takes its four steps s in one load)
     int2* late;          // [cols][C_in] later events {cin | bin << 16, alpha bits}
     int32_t* cnt;        // [cols] later events
@@ -82,22 +82,32 @@ __global__ __launch_bounds__(256) void k_split(SplitArgs a, int seg) {
     const int lane = lane_id(), wave = uniform(threadIdx.x >> 6);
     if (blockIdx.x == 0) {
         __shared__ float ths[kSplitMaxT + 1];
-        if (threadIdx.x <= kSplitMaxT) {
-            const int t = threadIdx.x;
-            const float th = t < a.T ? a.theta[t] : 0.0f;
+        for (int t = threadIdx.x; t <= kSplitMaxT; t += 256) {
+            const float th = a.theta && t < a.T ? a.theta[t] : 0.0f;
             ths[t] = (t < a.T && t >= a.t_min && th >= 1e-5f) ? th : __builtin_nanf("");
             if (t < kSplitMaxT) a.thr->th[t] = ths[t];
         }
         __syncthreads();
         if (threadIdx.x < 64) {
-            const float x0 = ths[lane], x1 = ths[64 + lane];
-            const uint64_t v0 = __ballot(x0 == x0), v1 = __ballot(x1 == x1);
-            const int lo = v0 ? __ffsll((unsigned long long)v0) - 1 : (v1 ? 63 + __ffsll((unsigned long long)v1) : 0);
-            const int hi = v1 ? 128 - __clzll((long long)v1) : (v0 ? 64 - __clzll((long long)v0) : 0);
+            int lo = kSplitMaxT, hi = 0;
+#pragma unroll
+            for (int k = 0; k < kSplitMaxT / 64; ++k) {
+                const float x = ths[64 * k + lane];
+                const uint64_t v = __ballot(x == x);
+                if (v != 0) {
+                    const int f = 64 * k + __ffsll((unsigned long long)v) - 1;
+                    lo = f < lo ? f : lo;
+                    hi = 64 * k + 64 - __clzll((long long)v);
+                }
+            }
+            lo = lo < hi ? lo : hi;
             // every step within [lo, hi) down or level (a NaN inside fails)
             bool down = true;
-            if (lane >= lo && lane < hi - 1) down = ths[lane] >= ths[lane + 1];
-            if (64 + lane >= lo && 64 + lane < hi - 1) down = down && ths[64 + lane] >= ths[64 + lane + 1];
+#pragma unroll
+            for (int k = 0; k < kSplitMaxT / 64; ++k) {
+                const int t = 64 * k + lane;
+                if (t >= lo && t < hi - 1) down = down && ths[t] >= ths[t + 1];
+            }
             const bool mono = __ballot(!down) == 0;
             if (lane == 0) {
                 const float l0 = hi > lo ? log2f(ths[lo]) : 0.0f, l1 = hi > lo ? log2f(ths[hi - 1]) : 0.0f;
@@ -127,9 +137,10 @@ __global__ __launch_bounds__(256) void k_split(SplitArgs a, int seg) {
             const float al = tb >= 0 ? lut[split_alpha(t, tb, a.alpha_by_time, a.T)] : 0.0f;
             const int g = (4 << a.hl) - 1;
             const int at = (ci & ~g) | ((ci & ((1 << a.hl) - 1)) << 2) | ((ci & g) >> a.hl);
-            if (cok && ci < a.Cp) a.a0[col * a.Cp + at] = tb == 0 ? al : 0.0f;
-            const uint64_t m = __ballot(tb > 0) & segm;
-            if (tb > 0) a.late[col * a.C_in + base + __popcll(m & lt)] = make_int2(ci | (tb << 16), __float_as_int(al));
+            if (a.a0 && cok && ci < a.Cp) a.a0[col * a.Cp + at] = tb == 0 ? al : 0.0f;
+            const bool listed = tb > 0 || (tb == 0 && !a.a0);
+            const uint64_t m = __ballot(listed) & segm;
+            if (listed) a.late[col * a.C_in + base + __popcll(m & lt)] = make_int2(ci | (tb << 16), __float_as_int(al));
             base += __popcll(m);
         }
         if (cok && r == 0) a.cnt[col] = base;
@@ -362,8 +373,14 @@ struct LateArgs {
     float tfs;
     int H_in, W_in, C_in, H_out, W_out, C_out, K_h, K_w, pad_h, pad_w;
     int rowbytes, w_bytes, cap, n_cblk, n_grp;
+    float decay, th;  // CuLIF
     FastDiv div_w, div_h;
 };
+
+// What k_late integrates: the later bins after k_gemm0's bin 0, or every bin
+// from the lists (k_split without bin-0 factors), with the LUT-threshold or the
+// CuLIF neuron.
+enum LateMode { kLateBins, kLateAll, kLateCulif };
 
 __host__ __device__ inline int late_entries(int cap) { return cap + kLatePad; }  // a multiple of 16
 // counts, cursors (64 TB each) and rank masks (128 TB) of one wave
@@ -440,7 +457,7 @@ __device__ __forceinline__ void slow_pixel(const LateArgs& a, int pix, int co) {
         if (ok[v]) a.out[(int64_t)pix * a.C_out + co + v] = res[v];
 }
 
-template <int GEO, int TB, bool TAPS9, bool W1>
+template <int GEO, int TB, bool TAPS9, bool W1, LateMode MODE>
 __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs a) {
     constexpr int OWN = 4 / GEO;  // c_out per lane
     constexpr int LPG = 8 / GEO;  // loads per group of 8 events
@@ -487,20 +504,20 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
 #pragma unroll
     for (int v = 0; v < OWN; ++v) {
         ok[v] = co + v < a.C_out;
-        carry[v] = ok[v] ? a.bias[co + v] : 0.0f;
-        acc[v] = ok[v] ? po[v] : 0.0f;
+        carry[v] = MODE != kLateCulif && ok[v] ? a.bias[co + v] : 0.0f;
+        acc[v] = MODE == kLateBins && ok[v] ? po[v] : 0.0f;
     }
     float v_th[TB];
     float* const tht = reinterpret_cast<float*>(tables + late_wave_words(TB) * W) + 2;  // thresholds, two NaN each side
 #pragma unroll
-    for (int k = 0; k < TB; ++k) v_th[k] = a.thr->th[64 * k + lane];
+    for (int k = 0; k < TB; ++k) v_th[k] = MODE != kLateCulif ? a.thr->th[64 * k + lane] : 0.0f;
     {
         const int z = vzero();
 #pragma unroll
         for (int i = 0; i < TB; ++i)  // counts, cursors, masks
             reinterpret_cast<int4*>(mine)[64 * i + lane] = make_int4(z, z, z, z);
     }
-    if (W1 || wave == 0) {
+    if (MODE != kLateCulif && (W1 || wave == 0)) {
 #pragma unroll
         for (int k = 0; k < TB; ++k) tht[64 * k + lane] = v_th[k];
         if (lane < 4) tht[lane < 2 ? lane - 2 : 64 * TB + lane - 2] = __builtin_nanf("");
@@ -525,6 +542,14 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
         e.x += k * a.C_in;  // row below 2^16 (host check)
         return e;
     };
+    if (MODE == kLateCulif && total == 0) {  // uniform over the workgroup
+        // no input: I and V stay 0, so a neuron fires at step 0 when 0 >= th
+        // (T3V:50-62) and never otherwise
+#pragma unroll
+        for (int v = 0; v < OWN; ++v)
+            if (cb < a.n_cblk && ok[v]) po[v] = 0.0f >= a.th ? 0.0f : kInfTime;
+        return;
+    }
     const int n_chunks = (total + 63) >> 6;
     const int c_lo = W1 ? 0 : (int)((unsigned)(n_chunks * wave) / (unsigned)W);
     const int c_hi = W1 ? n_chunks : (int)((unsigned)(n_chunks * (wave + 1)) / (unsigned)W);
@@ -621,8 +646,10 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
         res[v] = 0;
         alive[v] = __ballot(ok[v]);
     }
-    int b = 0;  // open bin, within its block of 64
-    bool second = false;
+    int blk = 0, b = 0;  // open bin: b within block blk of 64
+    float cur_i[OWN];     // the CuLIF current I
+#pragma unroll
+    for (int v = 0; v < OWN; ++v) cur_i[v] = 0.0f;
     float c_th = v_th[0];
     int c_end = v_end[0];
     int bend = __builtin_amdgcn_readlane(c_end, 0);
@@ -644,11 +671,27 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
             g.al[1] = *reinterpret_cast<const f4*>(alph + j + 4);
         }
     };
-    // closes one bin against the standing carries
+    auto next_block = [&]() __attribute__((always_inline)) {
+        ++blk;
+        b = 0;
+#pragma unroll
+        for (int k = 1; k < TB; ++k)
+            if (blk == k) {
+                c_th = v_th[k];
+                c_end = v_end[k];
+            }
+    };
+    // closes one bin: against the standing carries, or one CuLIF step with the
+    // bin's sum as its input (I = fma(I, decay, in); V += I)
     auto close_bin = [&]() __attribute__((always_inline)) {
-        const float th = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c_th), b));
+        const float th = MODE == kLateCulif ? a.th : __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c_th), b));
 #pragma unroll
         for (int v = 0; v < OWN; ++v) {
+            if constexpr (MODE == kLateCulif) {
+                cur_i[v] = __builtin_fmaf(cur_i[v], a.decay, acc[v]);
+                acc[v] = 0.0f;
+                carry[v] = carry[v] + cur_i[v];
+            }
             alive[v] &= ~__ballot(carry[v] >= th);
             res[v] = add_lane_bit(res[v], alive[v]);
         }
@@ -656,26 +699,20 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
     };
     // closes the bins before the one of the event at position p
     auto close_to = [&](int p) __attribute__((always_inline)) {
+        if constexpr (MODE != kLateCulif) {
 #pragma unroll
-        for (int v = 0; v < OWN; ++v) {
-            carry[v] = carry[v] + acc[v];
-            acc[v] = 0.0f;
+            for (int v = 0; v < OWN; ++v) {
+                carry[v] = carry[v] + acc[v];
+                acc[v] = 0.0f;
+            }
         }
         if constexpr (TB > 1) {
-            if (!second) {
+            for (;;) {
                 const int stop = __popcll(__builtin_amdgcn_ballot_w64(c_end <= p));
                 while (b < stop) close_bin();
-                if (b < 64) {
-                    bend = __builtin_amdgcn_readlane(c_end, b);
-                    return;
-                }
-                second = true;
-                b = 0;
-                c_th = v_th[TB - 1];
-                c_end = v_end[TB - 1];
+                if (b < 64) break;
+                next_block();
             }
-            const int stop = __popcll(__builtin_amdgcn_ballot_w64(c_end <= p));
-            while (b < stop) close_bin();
         } else {
             const int stop = __popcll(__builtin_amdgcn_ballot_w64(c_end <= p));
             do close_bin();
@@ -748,7 +785,7 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
         bool nan = false;
 #pragma unroll
         for (int v = 0; v < OWN; ++v) nan |= acc[v] != acc[v];
-        redo = live && __ballot(nan) != 0;
+        redo = MODE == kLateBins && live && __ballot(nan) != 0;
     }
     Raw g0, g1;
     int P0 = 0;
@@ -785,10 +822,31 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
         pad(P0);
         for (int c = c_lo; c < c_hi; ++c) place_chunk(element(c * 64 + lane), c * 64 + lane < total, P0);
         __syncthreads();
-        c_end = second ? v_end[TB - 1] : v_end[0];
+        c_end = v_end[0];
+#pragma unroll
+        for (int k = 1; k < TB; ++k)
+            if (blk == k) c_end = v_end[k];
         bend = __builtin_amdgcn_readlane(c_end, b);
     }
-    if (live) {
+    auto close_rest = [&]() __attribute__((always_inline)) {
+        for (;;) {
+            const int end = T - 64 * blk < 64 ? T - 64 * blk : 64;
+            while (b < end) {
+                close_bin();
+                if constexpr (MODE == kLateCulif) {
+                    uint64_t any = alive[0];
+#pragma unroll
+                    for (int v = 1; v < OWN; ++v) any |= alive[v];
+                    if (any == 0) return;
+                }
+            }
+            if (TB == 1 || 64 * blk + 64 >= T) return;
+            next_block();
+        }
+    };
+    if (MODE == kLateCulif) {
+        if (live) close_rest();  // every step without input steps the neuron too
+    } else if (live) {
         // The carries stand from the open bin on.  The first bin whose
         // threshold a carry reaches is guessed from the thresholds' slope and
         // taken where the thresholds around it bracket the carry; where one
@@ -797,7 +855,7 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
         // vector and 220 scalar instructions.
 #pragma unroll
         for (int v = 0; v < OWN; ++v) carry[v] = carry[v] + acc[v];
-        const int b0 = TB > 1 && second ? 64 + b : b;
+        const int b0 = 64 * blk + b;
         const int lo = a.thr->lo, hi = a.thr->hi;
         const float lg0 = a.thr->lg0, inv = a.thr->inv;
         bool bad = a.thr->mono == 0;
@@ -823,14 +881,7 @@ __global__ __launch_bounds__(W1 ? 64 : 64 * kLateMaxWaves) void k_late(LateArgs 
                 alive[v] &= ~fires[v];
             }
         } else {
-            while (b < 64 && (TB > 1 && second ? 64 : 0) + b < T) close_bin();
-            if constexpr (TB > 1) {
-                if (!second && T > 64) {
-                    b = 0;
-                    c_th = v_th[TB - 1];
-                    while (64 + b < T) close_bin();
-                }
-            }
+            close_rest();
         }
     }
     if (cb < a.n_cblk) {
@@ -867,7 +918,7 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
     const int T = ctx->c.T;
     const int taps = s.is_fc ? 1 : s.K_h * s.K_w;
     const int64_t cols = split_cols(s), pix = split_pix(s), K = (int64_t)taps * s.C_in;
-    if (T > kSplitMaxT || taps > kSplitMaxTaps || s.C_out < 32 || s.C_out > 16384) return false;
+    if (T > 128 || taps > kSplitMaxTaps || s.C_out < 32 || s.C_out > 16384) return false;
     // 16-bit weight rows in a list entry, row 0xFFFF past the weights; 32-bit buffer offsets
     if (K > 0xFFFF || K * s.C_out * 4 >= kOob) return false;
     if (cols * ceil16(s.C_in) * 4 >= kOob) return false;
@@ -896,6 +947,159 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
     return K * pix * s.C_out >= 100000000 || (K >= 1024 && s.C_out > 64);
 }
 
+// Layers the list form takes (k_split's lists with bin 0's events, then k_late
+// over every bin) in place of bucketize or dense merge, k_merge and k_stream:
+// windows past 64 steps, whose bins the fused kernels' lanes do not hold.
+// Measured, three launches to two: CuLIF 64->128 at 32x32, T = 160, batch 33:
+// 387 -> 190 us, 128->128 at 16x16: 321 -> 132; LeNet-5's FC layers at T = 80,
+// batch 128: 113 -> 51.  At T = 64 the fused kernels win: CuLIF 64->128 at
+// 128x128 2248 against 2460 us, LeNet-5's FC layers at batch 1024 45 against
+// 51.  Each group of four c_out blocks rebuilds a pixel's list and below 32
+// c_out a wave is mostly idle, so wide layers and narrow convolutions keep the
+// merged lists.
+bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
+    const int T = ctx->c.T;
+    const int taps = s.is_fc ? 1 : s.K_h * s.K_w;
+    const int64_t cols = split_cols(s), pix = split_pix(s), K = (int64_t)taps * s.C_in;
+    if (T > kSplitMaxT || taps > kSplitMaxTaps || s.C_out > 1024 || (s.C_out < 32 && !s.is_fc)) return false;
+    if (K > 0xFFFF || K * s.C_out * 4 >= kOob) return false;
+    if (cols * s.C_in * 4 >= kOob || pix * 8 >= (INT64_C(1) << 31)) return false;
+    return T > 64;
+}
+
+namespace {
+
+// k_late's launch over the lists in `late` and `cnt`.
+struct LateScratch {
+    int2* late;
+    int32_t* cnt;
+    LateThr* thr;
+};
+
+template <LateMode MODE>
+int launch_late(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const LateScratch& sc, const float* W,
+                const float* bias, const float* theta, int t_min, const IntegShape& s, const CulifNeuron* culif) {
+    const int taps = s.is_fc ? 1 : s.K_h * s.K_w;
+    const int64_t pix = split_pix(s);
+    LateArgs l{};
+    l.late = sc.late;
+    l.cnt = sc.cnt;
+    l.thr = sc.thr;
+    l.in = in;
+    l.alpha = alpha;
+    l.theta = theta;
+    l.bias = bias;
+    l.W = W;
+    l.out = out;
+    l.n_pix = (int)pix;
+    l.T = ctx->c.T;
+    l.t_min = t_min;
+    l.alpha_by_time = ctx->c.alpha_by_time;
+    l.tfs = ctx->c.tfs;
+    l.H_in = s.H_in;
+    l.W_in = s.W_in;
+    l.C_in = s.C_in;
+    l.H_out = s.H_out;
+    l.W_out = s.W_out;
+    l.C_out = s.C_out;
+    l.K_h = s.is_fc ? 1 : s.K_h;
+    l.K_w = s.is_fc ? 1 : s.K_w;
+    l.pad_h = s.pad_h;
+    l.pad_w = s.pad_w;
+    l.rowbytes = s.C_out * 4;
+    l.w_bytes = taps * s.C_in * s.C_out * 4;
+    l.div_w = make_fastdiv(s.W_out);
+    l.div_h = make_fastdiv(s.H_out);
+    if (culif) {
+        l.decay = culif->decay;
+        l.th = culif->th;
+    }
+    const int geo = s.C_out % 4 != 0 || s.C_out <= 64 ? 4 : 2;
+    const int cw = 256 / geo;
+    l.n_cblk = (s.C_out + cw - 1) / cw;
+    // waves that share a list: two keep an XCD's c_out group, and so the
+    // weights in its L2, small (VGG-16's 512-wide layers, four waves: 294 ->
+    // 311 us); the list form's longer lists are built by four
+    const int most = MODE == kLateBins ? 2 : kLateMaxWaves;
+    const int waves = l.n_cblk < most ? l.n_cblk : most;
+    l.n_grp = (l.n_cblk + waves - 1) / waves;
+    // list entries of a window: past the events of a usual field (later bins:
+    // a ninth of its elements in VGG-16), and LDS for 32 waves per CU
+    const int nel = taps * s.C_in;
+    const int nel_pad = (nel + 15) & ~15;
+    int cap = waves > 1 ? 640 : (nel > 1152 ? 512 : (MODE == kLateBins ? 192 : 320));
+    if (cap > nel_pad) cap = nel_pad;
+    l.cap = cap;
+    const int tb = l.T > 128 ? 4 : (l.T > 64 ? 2 : 1);
+    const size_t lds = (size_t)late_words(cap, waves, tb) * 4;
+    const int64_t lb = pix * l.n_grp;
+    if (lb > 0x7fffffff) return set_error(VDTTFS_E_UNSUPPORTED, "integrate: grid too large");
+#define VD_LATE(G, TBK, T9)                                                                                          \
+    do {                                                                                                             \
+        if (waves == 1)                                                                                              \
+            hipLaunchKernelGGL((k_late<G, TBK, T9, true, MODE>), dim3((unsigned)lb), dim3(64), lds, ctx->stream, l); \
+        else                                                                                                         \
+            hipLaunchKernelGGL((k_late<G, TBK, T9, false, MODE>), dim3((unsigned)lb), dim3(64 * waves), lds,         \
+                               ctx->stream, l);                                                                      \
+    } while (0)
+#define VD_LATE_T(G, TBK)           \
+    do {                            \
+        if (taps <= 9)              \
+            VD_LATE(G, TBK, true);  \
+        else                        \
+            VD_LATE(G, TBK, false); \
+    } while (0)
+#define VD_LATE_G(G)         \
+    do {                     \
+        if (tb == 1)         \
+            VD_LATE_T(G, 1); \
+        else if (tb == 2)    \
+            VD_LATE_T(G, 2); \
+        else if constexpr (MODE != kLateBins) \
+            VD_LATE_T(G, 4); \
+    } while (0)
+    if (geo == 4)
+        VD_LATE_G(4);
+    else
+        VD_LATE_G(2);
+#undef VD_LATE_G
+#undef VD_LATE_T
+#undef VD_LATE
+    VD_HIP(hipGetLastError());
+    return VDTTFS_OK;
+}
+
+int launch_split(vdttfs_ctx* ctx, const SplitArgs& k) {
+    int seg = 3;
+    while ((1 << seg) < k.Cp && seg < 6) ++seg;
+    const int64_t per_block = 4 * (64 >> seg);
+    int64_t blocks = (k.cols + per_block - 1) / per_block;
+    if (blocks > 8192) blocks = 8192;
+    hipLaunchKernelGGL(k_split, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, k, seg);
+    VD_HIP(hipGetLastError());
+    return VDTTFS_OK;
+}
+
+}  // namespace
+
+int launch_integrate_lists(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
+                           const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s,
+                           const CulifNeuron* culif) {
+    const int64_t cols = split_cols(s);
+    if (cols == 0 || split_pix(s) == 0) return VDTTFS_OK;
+    unsigned char* sp = static_cast<unsigned char*>(scratch);
+    LateScratch sc;
+    sc.late = reinterpret_cast<int2*>(sp);
+    sp += align256((size_t)cols * s.C_in * 8);
+    sc.cnt = reinterpret_cast<int32_t*>(sp);
+    sp += align256((size_t)cols * 4);
+    sc.thr = reinterpret_cast<LateThr*>(sp);
+    VD_TRY(launch_split(ctx, SplitArgs{in, nullptr, sc.late, sc.cnt, alpha, theta, sc.thr, cols, s.C_in, s.C_in,
+                                       ctx->c.T, ctx->c.alpha_by_time, t_min, 1, ctx->c.tfs}));
+    if (culif) return launch_late<kLateCulif>(ctx, out, in, alpha, sc, W, bias, theta, t_min, s, culif);
+    return launch_late<kLateAll>(ctx, out, in, alpha, sc, W, bias, theta, t_min, s, nullptr);
+}
+
 int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
                            const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s) {
     const int64_t cols = split_cols(s), pix = split_pix(s);
@@ -907,21 +1111,14 @@ int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const f
     unsigned char* sp = static_cast<unsigned char*>(scratch);
     float* a0 = reinterpret_cast<float*>(sp);
     sp += align256((size_t)cols * ceil16(s.C_in) * 4);
-    int2* late = reinterpret_cast<int2*>(sp);
+    LateScratch sc;
+    sc.late = reinterpret_cast<int2*>(sp);
     sp += align256((size_t)cols * s.C_in * 8);
-    int32_t* cnt = reinterpret_cast<int32_t*>(sp);
+    sc.cnt = reinterpret_cast<int32_t*>(sp);
     sp += align256((size_t)cols * 4);
-    LateThr* thr = reinterpret_cast<LateThr*>(sp);
-
-    const SplitArgs k{in,   a0, late,      cnt, alpha,                 theta, thr,
-                      cols, s.C_in, Cp, ctx->c.T, ctx->c.alpha_by_time, t_min, mf == 16 ? 2 : 1, ctx->c.tfs};
-    int seg = 3;
-    while ((1 << seg) < Cp && seg < 6) ++seg;
-    const int64_t per_block = 4 * (64 >> seg);
-    int64_t blocks = (cols + per_block - 1) / per_block;
-    if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL(k_split, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, k, seg);
-    VD_HIP(hipGetLastError());
+    sc.thr = reinterpret_cast<LateThr*>(sp);
+    VD_TRY(launch_split(ctx, SplitArgs{in, a0, sc.late, sc.cnt, alpha, theta, sc.thr, cols, s.C_in, Cp, ctx->c.T,
+                                       ctx->c.alpha_by_time, t_min, mf == 16 ? 2 : 1, ctx->c.tfs}));
 
     Gemm0Args g{};
     g.a0 = a0;
@@ -971,82 +1168,7 @@ int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const f
 #undef VD_GEMM0
     VD_HIP(hipGetLastError());
 
-    LateArgs l{};
-    l.late = late;
-    l.cnt = cnt;
-    l.in = in;
-    l.alpha = alpha;
-    l.theta = theta;
-    l.thr = thr;
-    l.bias = bias;
-    l.W = W;
-    l.out = out;
-    l.n_pix = (int)pix;
-    l.T = ctx->c.T;
-    l.t_min = t_min;
-    l.alpha_by_time = ctx->c.alpha_by_time;
-    l.tfs = ctx->c.tfs;
-    l.H_in = s.H_in;
-    l.W_in = s.W_in;
-    l.C_in = s.C_in;
-    l.H_out = s.H_out;
-    l.W_out = s.W_out;
-    l.C_out = s.C_out;
-    l.K_h = g.K_h;
-    l.K_w = g.K_w;
-    l.pad_h = s.pad_h;
-    l.pad_w = s.pad_w;
-    l.rowbytes = g.rowbytes;
-    l.w_bytes = g.w_bytes;
-    l.div_w = g.div_w;
-    l.div_h = g.div_h;
-    const int geo = s.C_out % 4 != 0 || s.C_out <= 64 ? 4 : 2;
-    const int cw = 256 / geo;
-    l.n_cblk = (s.C_out + cw - 1) / cw;
-    const int waves = l.n_cblk < 2 ? l.n_cblk : 2;
-    l.n_grp = (l.n_cblk + waves - 1) / waves;
-    const int nel = taps * s.C_in;
-    const int tb = l.T > 64 ? 2 : 1;
-    // list entries of a window: past the events of a usual field (a ninth of
-    // its elements in VGG-16), and LDS for 32 waves per CU
-    const int nel_pad = (nel + 15) & ~15;
-    int cap = waves > 1 ? 640 : (nel > 1152 ? 512 : 192);
-    if (cap > nel_pad) cap = nel_pad;
-    l.cap = cap;
-    const size_t lds = (size_t)late_words(cap, waves, tb) * 4;
-    const int64_t lb = pix * l.n_grp;
-    if (lb > 0x7fffffff) return set_error(VDTTFS_E_UNSUPPORTED, "integrate: grid too large");
-#define VD_LATE(G, TBK, T9)                                                                                         \
-    do {                                                                                                            \
-        if (waves == 1)                                                                                             \
-            hipLaunchKernelGGL((k_late<G, TBK, T9, true>), dim3((unsigned)lb), dim3(64), lds, ctx->stream, l);      \
-        else                                                                                                        \
-            hipLaunchKernelGGL((k_late<G, TBK, T9, false>), dim3((unsigned)lb), dim3(64 * waves), lds, ctx->stream, \
-                               l);                                                                                  \
-    } while (0)
-#define VD_LATE_T(G, TBK)          \
-    do {                           \
-        if (taps <= 9)             \
-            VD_LATE(G, TBK, true); \
-        else                       \
-            VD_LATE(G, TBK, false);\
-    } while (0)
-#define VD_LATE_G(G)         \
-    do {                     \
-        if (tb == 1)         \
-            VD_LATE_T(G, 1); \
-        else                 \
-            VD_LATE_T(G, 2); \
-    } while (0)
-    if (geo == 4)
-        VD_LATE_G(4);
-    else
-        VD_LATE_G(2);
-#undef VD_LATE_G
-#undef VD_LATE_T
-#undef VD_LATE
-    VD_HIP(hipGetLastError());
-    return VDTTFS_OK;
+    return launch_late<kLateBins>(ctx, out, in, alpha, sc, W, bias, theta, t_min, s, nullptr);
 }
 
 }  // namespace vdttfs

@@ -254,8 +254,8 @@ int forward_impl(vdttfs_net* net, const float* d_img, int32_t* d_pred, uint64_t*
             // and in a counting forward for its retained-event count
             LaunchPlan plan;
             VD_TRY(resolve_plan(ctx, s, l.plan, &plan));
-            // the built-in choice of a layer with a late fire start; its scratch
-            // is the merged lists' (sized for both at creation)
+            // the built-in choice of layers with a late fire start or a long
+            // window; its scratch is the merged lists' (sized for both at creation)
             const bool split = plan.split && !count && !fuse;
             const bool dense = split || plan_from_dense(ctx, s, plan, count);
             TimedPair tb{}, ti{};
@@ -273,7 +273,10 @@ int forward_impl(vdttfs_net* net, const float* d_img, int32_t* d_pred, uint64_t*
             } else if (net->timing) {
                 VD_TRY(mark(net, &ti.a));
             }
-            if (split)
+            if (split && plan.split == kSplitLists)
+                VD_TRY(launch_integrate_lists(ctx, l.out, cur, l.alpha, net->list, l.W, l.bias, l.theta, l.t_min, s,
+                                              nullptr));
+            else if (split)
                 VD_TRY(launch_integrate_split(ctx, l.out, cur, l.alpha, net->list, l.W, l.bias, l.theta, l.t_min, s));
             else if (dense)
                 VD_TRY(launch_integrate_dense(ctx, l.out, cur, l.alpha, net->list, l.list_cap,
@@ -405,7 +408,7 @@ int create_impl(vdttfs_net* net, const vdttfs_layer_desc* layers, int n) {
         const int64_t n_pix = (int64_t)net->B * (fc ? 1 : (int64_t)d.H_out * d.W_out);
         if (n_pix * l.list_cap > max_list) max_list = n_pix * l.list_cap;
         const int64_t split_list = (int64_t)(split_scratch_bytes(s) / sizeof(int2)) + 1;
-        if (c.tfs > 0.0f && split_list > max_list) max_list = split_list;
+        if ((c.tfs > 0.0f || c.T > 64) && split_list > max_list) max_list = split_list;
         if (n_pix * (c.T + 1) > max_bstart) max_bstart = n_pix * (c.T + 1);
     }
     for (int i = 0; i < n; ++i) net->L[i].d.kernel = net->L[i].d.bias = nullptr;
