@@ -259,12 +259,19 @@ struct StepLayer {
     int64_t n;  // neurons: B * H_out * W_out * C_out
     int H_in, W_in, C_in, H_out, W_out, C_out, K_h, K_w, pad_h, pad_w, is_fc;
 };
-int launch_step_input(vdttfs_ctx* ctx, const float* tin, uint8_t* s, int64_t n, int t);
-int launch_step_neuron(vdttfs_ctx* ctx, const StepLayer& L, const uint8_t* s_in, uint8_t* s_out, float* vmem,
-                       uint8_t* fired, float* out, int mode, int int_ok, int fire_ok, int out_layer, float kv,
-                       float th, int t);
-int launch_step_pool(vdttfs_ctx* ctx, const uint8_t* s_in, uint8_t* s_out, uint8_t* fired, int64_t n, int H_in,
-                     int W_in, int C);
+// A layer's steps: it integrates at n_int steps from t0 on (decay kv) and may
+// fire at those where th is not NaN, then, its potential standing, at
+// the n_after steps from t_after on where th_after is not NaN.
+constexpr int kStepMaxWin = 256;  // a window's steps (T <= 255, and one for a fractional fire start)
+struct StepWindows {
+    float t0 = 0.0f, t_after = 0.0f;
+    int n_int = 0, n_after = 0;
+    int out_layer = 0;  // T1S: no spike is 9999; T2S: keeps max(V + b) instead of firing
+    float kv[kStepMaxWin] = {}, th[kStepMaxWin], th_after[kStepMaxWin];
+};
+int launch_step_layer(vdttfs_ctx* ctx, const StepLayer& L, const float* in, float* out, int mode,
+                      const StepWindows& w);
+int launch_step_pool(vdttfs_ctx* ctx, const float* in, float* out, int64_t n, int H_in, int W_in, int C, int steps);
 int launch_step_fill(vdttfs_ctx* ctx, float* p, int64_t n, float v);
 
 // Step-by-step CuLIF baseline (T3S semantics): one layer of the time-driven

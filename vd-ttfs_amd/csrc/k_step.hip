@@ -1,129 +1,171 @@
 // Step-by-step (time-driven) baseline kernels: the reference's own GPU
 // denominator (T1S = task1_lenet_mnist/stepbystep_cuda/snn_mnist_stepbystep.cu,
-// T2S = task2_vgg16_cifar10/stepbystep_cuda/bench_vgg_timedriven_baseline.cu),
-// rebuilt for gfx950 with the reference's work structure: every global step
-// launches every layer, one thread per neuron scans its whole receptive field
-// for inputs that spike at that step, and neurons fire once on the decaying
-// threshold.  No event lists and no early exit: this is the baseline the
-// event-driven engine is measured against.
-//   k_step_input  input spikes of step t from the encoded first-spike times;
-//   k_step_neuron conv / FC step (T1S:47-103, T2S:53-108 and 141-200);
+// T2S = task2_vgg16_cifar10/stepbystep_cuda/bench_vgg_timedriven_baseline.cu):
+// every neuron takes every step of its windows, scans its whole receptive
+// field (no event lists), and fires once on the decaying threshold.
+//   k_step_layer  conv / FC layer, all its steps (T1S:47-103, T2S:53-108 and
+//                 141-200);
 //   k_step_pool   spiking 2x2 pool (T1S:107-127, T2S:110-139);
-//   k_s3_*        the CuLIF network of T3S (below).
+//   k_s3_*        the CuLIF network of T3S (below), a launch per layer and step.
+// T1S and T2S launch every layer at every step; their neurons spike at most
+// once and feed forward only, so a layer's spikes of all steps are its
+// first-spike steps, and the layers run one after the other, each over all
+// steps, with the state of a neuron in registers in between.
 // The step's decay kv(t) and threshold th(t) are the same for every neuron of
 // a layer; the host evaluates them once per (layer, step) with the same expf
-// expressions and passes them in.  Threads are numbered c_out fastest, so a
-// wave's threads read the same input spikes and consecutive weights.
+// expressions and passes them in.
 #include "common.h"
 #include "wave.h"
 
 namespace vdttfs {
 namespace {
 
-__global__ __launch_bounds__(256) void k_step_input(const float* __restrict__ tin, uint8_t* __restrict__ s,
-                                                    int64_t n, float t) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        s[i] = tin[i] == t ? 1 : 0;
-}
+// One thread per neuron (numbered c_out fastest, so a wave's threads read the
+// same inputs and consecutive weights), one wave per workgroup.  A thread scans
+// its field once, in (kh, kw, c_in) order, and adds each input that spikes to
+// the sum of its step, one LDS column of n_int steps per thread: a step's sum
+// is the same chain, in the same order, as a scan of the field at that step.
+// Then the thread runs the steps.  Bound by latency: the read-modify-write of
+// the LDS column per spike and the loads of the scan, with ten waves on a CU
+// (16 KB of LDS each at 64 steps); 16 inputs and weights are loaded ahead of
+// the chain, and a wave's place in the field is kept in scalar registers.
+// LeNet-5, T = 64, batch 256: 520 launches that read the field and the state
+// of every neuron T times took 3126 us, these nine take 124 (conv1 71 us,
+// conv2 64, the FC layers 78 when each runs alone).
+constexpr int kStepAhead = 16;
 
 struct StepArgs {
-    const uint8_t* s_in;
-    uint8_t* s_out;
-    float* vmem;
-    uint8_t* fired;
+    const float* in;   // first-spike steps of the inputs (no step: does not spike)
+    float* out;        // first-spike steps, else +inf (T1S output: 9999); T2S output layer: max(V + b)
     const float* W;
     const float* bias;
-    float* out;  // output layer: first-spike steps (T1S) or max(V + b) (T2S)
     int64_t n;
-    int H_in, W_in, C_in, H_out, W_out, C_out, K_h, K_w, pad_h, pad_w, is_fc;
-    int mode;          // 1: T1S (psp = sum w; V = fma(psp, kv, V)); 2: T2S (psp = fma chain of w*kv; V += psp)
-    int int_ok, fire_ok;
-    int out_layer;     // 1: T1S output (records its first spike); 2: T2S output (keeps max V + b)
-    float kv, th, t;
+    int H_in, W_in, C_in, H_out, W_out, C_out, K_h, K_w, pad_h, pad_w;
+    StepWindows w;
 };
 
-__global__ __launch_bounds__(256) void k_step_neuron(StepArgs a) {
-    for (int64_t nid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; nid < a.n;
-         nid += (int64_t)gridDim.x * blockDim.x) {
-        const bool keep_max = a.out_layer == 2;
-        if (!keep_max && a.fired[nid]) {
-            a.s_out[nid] = 0;
-            continue;
-        }
-        const int co = (int)(nid % a.C_out);
-        float V = a.vmem[nid];
-        if (a.int_ok) {
-            float psp = 0.0f;
-            if (a.is_fc) {
-                const int cin = a.H_in * a.W_in * a.C_in;
-                const uint8_t* src = a.s_in + (nid / a.C_out) * cin;
-                for (int ci = 0; ci < cin; ++ci)
-                    if (src[ci]) {
-                        const float w = a.W[(int64_t)ci * a.C_out + co];
-                        psp = a.mode == 1 ? psp + w : __builtin_fmaf(w, a.kv, psp);
-                    }
+// PAD: taps may fall outside the map.
+template <int MODE, bool PAD>  // 1: T1S (psp = sum w; V = fma(psp, kv, V)); 2: T2S (psp = fma chain of w*kv; V += psp)
+__global__ __launch_bounds__(64) void k_step_layer(StepArgs a) {
+    extern __shared__ float lds[];
+    const int lane = threadIdx.x;
+    const int n_int = a.w.n_int, n_pad = (n_int + 7) & ~7;
+    float* const psp = lds + lane;  // step t0 + s at psp[64 s]; read and written by this thread alone
+    for (int s = 0; s < n_pad; s += 8)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) psp[64 * (s + k)] = 0.0f;
+    float kvr[kStepMaxWin / 64];  // T2S: kv of step 64 k + lane
+#pragma unroll
+    for (int k = 0; k < kStepMaxWin / 64; ++k) kvr[k] = MODE == 2 ? a.w.kv[64 * k + lane] : 0.0f;
+    const int64_t nid_raw = (int64_t)blockIdx.x * 64 + lane;
+    const bool real = nid_raw < a.n;
+    const int64_t nid = real ? nid_raw : a.n - 1;
+    const int64_t q = nid / a.C_out;
+    const int co = (int)(nid - q * a.C_out);
+    const int wo = (int)(q % a.W_out);
+    const int ho = (int)((q / a.W_out) % a.H_out);
+    const int64_t img = q / ((int64_t)a.W_out * a.H_out);
+    const int h0 = ho - a.pad_h, w0 = wo - a.pad_w;
+    const float* const src = a.in + img * a.H_in * a.W_in * a.C_in;
+    const float* const tap0 = src + ((int64_t)h0 * a.W_in + w0) * a.C_in;  // tap (0, 0); read inside the map only
+    const int K = a.K_h * a.K_w * a.C_in;
+    const int64_t row = (int64_t)(a.W_in - a.K_w) * a.C_in;  // from a row's last tap to the next row's first
+    // the next element, the same in every lane: its place, its distance from
+    // tap (0, 0) and its weights
+    int kh = 0, kw = 0, ci = 0;
+    int64_t off = 0;
+    const float* wt = a.W;
+    for (int e0 = 0; e0 < K; e0 += kStepAhead) {
+        float x[kStepAhead], w[kStepAhead];
+#pragma unroll
+        for (int u = 0; u < kStepAhead; ++u) {
+            const bool in_field = e0 + u < K;  // past the last element: the last one again, as no input
+            bool ok = in_field;
+            if constexpr (PAD) {
+                ok = ok && (unsigned)(h0 + kh) < (unsigned)a.H_in && (unsigned)(w0 + kw) < (unsigned)a.W_in;
+                x[u] = *(ok ? tap0 + off : src);
             } else {
-                const int64_t q = nid / a.C_out;
-                const int wo = (int)(q % a.W_out);
-                const int ho = (int)((q / a.W_out) % a.H_out);
-                const int64_t img = q / ((int64_t)a.W_out * a.H_out);
-                for (int kh = 0; kh < a.K_h; ++kh) {
-                    const int hi = ho - a.pad_h + kh;
-                    if (hi < 0 || hi >= a.H_in) continue;
-                    for (int kw = 0; kw < a.K_w; ++kw) {
-                        const int wi = wo - a.pad_w + kw;
-                        if (wi < 0 || wi >= a.W_in) continue;
-                        const uint8_t* src = a.s_in + ((img * a.H_in + hi) * a.W_in + wi) * a.C_in;
-                        const int64_t wb = (int64_t)(kh * a.K_w + kw) * a.C_in;
-                        for (int ci = 0; ci < a.C_in; ++ci)
-                            if (src[ci]) {
-                                const float w = a.W[(wb + ci) * a.C_out + co];
-                                psp = a.mode == 1 ? psp + w : __builtin_fmaf(w, a.kv, psp);
-                            }
+                x[u] = tap0[off];
+            }
+            if (!ok) x[u] = -1.0f;
+            w[u] = wt[co];
+            if (e0 + u + 1 < K) {
+                ++off;
+                wt += a.C_out;
+                if (++ci == a.C_in) {
+                    ci = 0;
+                    if (++kw == a.K_w) {
+                        kw = 0;
+                        ++kh;
+                        off += row;
                     }
                 }
             }
-            V = a.mode == 1 ? __builtin_fmaf(psp, a.kv, V) : V + psp;
-            a.vmem[nid] = V;
         }
-        uint8_t spike = 0;
-        if (keep_max) {
-            if (a.int_ok) {
-                const float v = V + a.bias[co];
-                if (v > a.out[nid]) a.out[nid] = v;
+#pragma unroll
+        for (int u = 0; u < kStepAhead; ++u) {
+            // an input spikes at step t where its time equals t
+            const float d = x[u] - a.w.t0;
+            const bool ev = d >= 0.0f && d < (float)n_int && x[u] == floorf(x[u]);
+            const int s = ev ? (int)d : 0;
+            float kv = 0.0f;
+            if constexpr (MODE == 2) {
+                kv = __shfl(kvr[0], s & 63, 64);
+#pragma unroll
+                for (int k = 1; k < kStepMaxWin / 64; ++k)
+                    if (64 * k < n_int) {  // uniform
+                        const float y = __shfl(kvr[k], s & 63, 64);
+                        kv = (s >> 6) == k ? y : kv;
+                    }
             }
-        } else if (a.fire_ok && V + a.bias[co] >= a.th && a.th >= 1e-5f) {
-            spike = 1;
-            a.fired[nid] = 1;
-            if (a.out_layer == 1 && a.out[nid] >= kInfTime) a.out[nid] = a.t;
+            if (ev) psp[64 * s] = MODE == 1 ? psp[64 * s] + w[u] : __builtin_fmaf(w[u], kv, psp[64 * s]);
         }
-        a.s_out[nid] = spike;
     }
+    const float b = a.bias[co];
+    float V = 0.0f;
+    // the steps, 8 sums and their constants loaded at a time (those past the
+    // last add nothing and cannot fire)
+    float first = __builtin_inff(), best = -1e9f;
+    for (int s0 = 0; s0 < n_pad; s0 += 8) {
+        float p[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) p[k] = psp[64 * (s0 + k)];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            // a neuron that has fired integrates on: nothing reads its V then
+            V = MODE == 1 ? __builtin_fmaf(p[k], a.w.kv[s0 + k], V) : V + p[k];
+            const float v = V + b;
+            if (MODE == 2 && a.w.out_layer)
+                best = v > best ? v : best;
+            else if (first == __builtin_inff() && v >= a.w.th[s0 + k])
+                first = a.w.t0 + (float)(s0 + k);
+        }
+    }
+    if (MODE == 2 && a.w.out_layer) {
+        if (real) a.out[nid] = best;
+        return;
+    }
+    for (int s = 0; s < a.w.n_after; ++s)
+        if (first == __builtin_inff() && V + b >= a.w.th_after[s]) first = a.w.t_after + (float)s;
+    if (a.w.out_layer && first == __builtin_inff()) first = kInfTime;
+    if (real) a.out[nid] = first;
 }
 
-__global__ __launch_bounds__(256) void k_step_pool(const uint8_t* __restrict__ s_in, uint8_t* __restrict__ s_out,
-                                                   uint8_t* __restrict__ fired, int64_t n, int H_in, int W_in,
-                                                   int C) {
+// A pool neuron spikes with the first spike of its window.
+__global__ __launch_bounds__(256) void k_step_pool(const float* __restrict__ in, float* __restrict__ out, int64_t n,
+                                                   int H_in, int W_in, int C, float steps) {
     const int Ho = H_in / 2, Wo = W_in / 2;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
          idx += (int64_t)gridDim.x * blockDim.x) {
-        if (fired[idx]) {
-            s_out[idx] = 0;
-            continue;
-        }
         const int c = (int)(idx % C), w = (int)((idx / C) % Wo), h = (int)((idx / C / Wo) % Ho);
         const int64_t b = idx / ((int64_t)C * Wo * Ho);
-        uint8_t spike = 0;
-        for (int i = 0; i < 2 && !spike; ++i)
-            for (int j = 0; j < 2; ++j) {
-                const int hi = h * 2 + i, wi = w * 2 + j;
-                if (hi < H_in && wi < W_in && s_in[((b * H_in + hi) * W_in + wi) * C + c]) {
-                    spike = 1;
-                    break;
-                }
-            }
-        if (spike) fired[idx] = 1;
-        s_out[idx] = spike;
+        float m = __builtin_inff();
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float x = in[((b * H_in + 2 * h + k / 2) * W_in + 2 * w + k % 2) * C + c];
+            if (x >= 0.0f && x < steps && x == floorf(x)) m = fminf(m, x);
+        }
+        out[idx] = m;
     }
 }
 
@@ -140,51 +182,47 @@ unsigned step_grid(int64_t n) {
 
 }  // namespace
 
-int launch_step_input(vdttfs_ctx* ctx, const float* tin, uint8_t* s, int64_t n, int t) {
-    hipLaunchKernelGGL(k_step_input, dim3(step_grid(n)), dim3(256), 0, ctx->stream, tin, s, n, (float)t);
-    VD_HIP(hipGetLastError());
-    return VDTTFS_OK;
-}
-
-int launch_step_neuron(vdttfs_ctx* ctx, const StepLayer& L, const uint8_t* s_in, uint8_t* s_out, float* vmem,
-                       uint8_t* fired, float* out, int mode, int int_ok, int fire_ok, int out_layer, float kv,
-                       float th, int t) {
+int launch_step_layer(vdttfs_ctx* ctx, const StepLayer& L, const float* in, float* out, int mode,
+                      const StepWindows& w) {
+    if (L.n == 0) return VDTTFS_OK;
+    if (w.n_int < 0 || w.n_int > kStepMaxWin || w.n_after < 0 || w.n_after > kStepMaxWin)
+        return set_error(VDTTFS_E_UNSUPPORTED, "step layer: windows of %d and %d steps", w.n_int, w.n_after);
     StepArgs a{};
-    a.s_in = s_in;
-    a.s_out = s_out;
-    a.vmem = vmem;
-    a.fired = fired;
+    a.in = in;
+    a.out = out;
     a.W = L.W;
     a.bias = L.bias;
-    a.out = out;
     a.n = L.n;
-    a.H_in = L.H_in;
-    a.W_in = L.W_in;
-    a.C_in = L.C_in;
-    a.H_out = L.H_out;
-    a.W_out = L.W_out;
+    a.H_in = L.is_fc ? 1 : L.H_in;
+    a.W_in = L.is_fc ? 1 : L.W_in;
+    a.C_in = L.is_fc ? L.H_in * L.W_in * L.C_in : L.C_in;
+    a.H_out = L.is_fc ? 1 : L.H_out;
+    a.W_out = L.is_fc ? 1 : L.W_out;
     a.C_out = L.C_out;
-    a.K_h = L.K_h;
-    a.K_w = L.K_w;
-    a.pad_h = L.pad_h;
-    a.pad_w = L.pad_w;
-    a.is_fc = L.is_fc;
-    a.mode = mode;
-    a.int_ok = int_ok;
-    a.fire_ok = fire_ok;
-    a.out_layer = out_layer;
-    a.kv = kv;
-    a.th = th;
-    a.t = (float)t;
-    hipLaunchKernelGGL(k_step_neuron, dim3(step_grid(L.n)), dim3(256), 0, ctx->stream, a);
+    a.K_h = L.is_fc ? 1 : L.K_h;
+    a.K_w = L.is_fc ? 1 : L.K_w;
+    a.pad_h = L.is_fc ? 0 : L.pad_h;
+    a.pad_w = L.is_fc ? 0 : L.pad_w;
+    a.w = w;
+    const int64_t blocks = (L.n + 63) / 64;
+    if (blocks > 0x7fffffff) return set_error(VDTTFS_E_UNSUPPORTED, "step layer: grid too large");
+    const size_t lds = (size_t)64 * ((w.n_int + 7) & ~7) * 4;
+    const bool pad = a.pad_h != 0 || a.pad_w != 0;
+    if (mode == 1 && pad)
+        hipLaunchKernelGGL((k_step_layer<1, true>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
+    else if (mode == 1)
+        hipLaunchKernelGGL((k_step_layer<1, false>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
+    else if (pad)
+        hipLaunchKernelGGL((k_step_layer<2, true>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
+    else
+        hipLaunchKernelGGL((k_step_layer<2, false>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
     VD_HIP(hipGetLastError());
     return VDTTFS_OK;
 }
 
-int launch_step_pool(vdttfs_ctx* ctx, const uint8_t* s_in, uint8_t* s_out, uint8_t* fired, int64_t n, int H_in,
-                     int W_in, int C) {
-    hipLaunchKernelGGL(k_step_pool, dim3(step_grid(n)), dim3(256), 0, ctx->stream, s_in, s_out, fired, n, H_in,
-                       W_in, C);
+int launch_step_pool(vdttfs_ctx* ctx, const float* in, float* out, int64_t n, int H_in, int W_in, int C, int steps) {
+    hipLaunchKernelGGL(k_step_pool, dim3(step_grid(n)), dim3(256), 0, ctx->stream, in, out, n, H_in, W_in, C,
+                       (float)steps);
     VD_HIP(hipGetLastError());
     return VDTTFS_OK;
 }

@@ -1,10 +1,11 @@
 // Step-by-step (time-driven) baseline network (T1S / T2S main loops,
-// T1S:222-244 and T2S:329-352): encode once, then for every global step the
-// input spikes of that step and every layer in order, then the readout.
+// T1S:222-244 and T2S:329-352): encode once, then every layer over all the
+// global steps (k_step.hip says why the order of layers and steps may turn),
+// then the readout.
 // T3S mode (snn_dvs_stepbystep.cu:220-252) steps the CuLIF layer table over
 // the dense event tensor.
-// Weights are uploaded once; spike maps, membrane potentials and fire-once
-// latches live on the device for the batch.
+// Weights are uploaded once; the layers' first-spike steps live on the device
+// for the batch.
 #include <cmath>
 #include <new>
 #include <vector>
@@ -21,9 +22,7 @@ struct StepNetLayer {
     int depth = 0;                    // 1-based among weighted layers
     float* W = nullptr;
     float* bias = nullptr;
-    uint8_t* spk = nullptr;
-    uint8_t* fired = nullptr;
-    float* vmem = nullptr;
+    float* first = nullptr;  // first-spike steps
 };
 
 struct vdttfs_stepnet {
@@ -33,7 +32,6 @@ struct vdttfs_stepnet {
     float tc_in = 16.0f, td_in = 0.0f;
     std::vector<StepNetLayer> L;
     float* tin = nullptr;  // encoded first-spike times of the input
-    uint8_t* s0 = nullptr;
     float* out = nullptr;
     int64_t out_elems = 0;
     // T3S mode: the CuLIF layers and every buffer they own
@@ -50,10 +48,9 @@ void release(vdttfs_stepnet* net) {
         (void)hipStreamSynchronize(net->ctx->stream);
     }
     for (StepNetLayer& l : net->L)
-        for (void* p : {(void*)l.W, (void*)l.bias, (void*)l.spk, (void*)l.fired, (void*)l.vmem})
+        for (void* p : {(void*)l.W, (void*)l.bias, (void*)l.first})
             if (p) (void)hipFree(p);
-    for (void* p : {(void*)net->tin, (void*)net->s0})
-        if (p) (void)hipFree(p);
+    if (net->tin) (void)hipFree(net->tin);
     if (net->mode != VDTTFS_STEP_T3 && net->out) (void)hipFree(net->out);  // T3S: out is a layer's ft
     for (void* p : net->bufs3)
         if (p) (void)hipFree(p);
@@ -78,7 +75,6 @@ int create_impl(vdttfs_stepnet* net, const vdttfs_layer_desc* layers, int n) {
     vdttfs_ctx* ctx = net->ctx;
     const vdttfs_consts& c = ctx->c;
     VD_TRY(dmalloc((void**)&net->tin, (size_t)net->B * net->img_elems * 4));
-    VD_TRY(dmalloc((void**)&net->s0, (size_t)net->B * net->img_elems));
     net->L.resize(n);
     float tc = net->tc_in, td = net->td_in;
     int depth = 0;
@@ -100,14 +96,12 @@ int create_impl(vdttfs_stepnet* net, const vdttfs_layer_desc* layers, int n) {
         const bool same = !s.is_fc && c.conv_same_pad;  // T2V:109-110
         s.pad_h = same ? d.K_h / 2 : 0;
         s.pad_w = same ? d.K_w / 2 : 0;
-        VD_TRY(dmalloc((void**)&l.spk, (size_t)s.n));
-        VD_TRY(dmalloc((void**)&l.fired, (size_t)s.n));
+        if (i != n - 1) VD_TRY(dmalloc((void**)&l.first, (size_t)s.n * 4));
         if (d.kind == VDTTFS_LAYER_POOL) continue;
         const int64_t kel = s.is_fc ? (int64_t)d.H_in * d.W_in * d.C_in * d.C_out
                                     : (int64_t)d.K_h * d.K_w * d.C_in * d.C_out;
         VD_TRY(upload(&l.W, d.kernel, (size_t)kel));
         VD_TRY(upload(&l.bias, d.bias, (size_t)d.C_out));
-        VD_TRY(dmalloc((void**)&l.vmem, (size_t)s.n * 4));
         s.W = l.W;
         s.bias = l.bias;
         l.tc_i = tc;
@@ -135,22 +129,20 @@ int forward_impl(vdttfs_stepnet* net, const float* d_img, int32_t* d_pred) {
         VD_TRY(launch_encode_log(ctx, d_img, net->tin, n_img, net->tc_in, net->td_in));
     else
         VD_TRY(launch_encode_linear(ctx, d_img, net->tin, n_img));
-    for (StepNetLayer& l : net->L) {
-        VD_HIP(hipMemsetAsync(l.fired, 0, (size_t)l.s.n, ctx->stream));
-        if (l.vmem) VD_TRY(launch_step_fill(ctx, l.vmem, l.s.n, 0.0f));
-    }
     const bool t1 = net->mode == VDTTFS_STEP_T1;
-    VD_TRY(launch_step_fill(ctx, net->out, net->out_elems, t1 ? kInfTime : -1e9f));
     const int last = (int)net->L.size() - 1;
-    for (int t = 0; t < net->steps; ++t) {
-        VD_TRY(launch_step_input(ctx, net->tin, net->s0, n_img, t));
-        const uint8_t* s_in = net->s0;
-        for (int i = 0; i <= last; ++i) {
-            StepNetLayer& l = net->L[i];
-            if (l.s.kind == VDTTFS_LAYER_POOL) {
-                VD_TRY(launch_step_pool(ctx, s_in, l.spk, l.fired, l.s.n, l.s.H_in, l.s.W_in, l.s.C_in));
-            } else {
-                int int_ok, fire_ok;
+    const float* in = net->tin;
+    for (int i = 0; i <= last; ++i) {
+        StepNetLayer& l = net->L[i];
+        float* out = i == last ? net->out : l.first;
+        if (l.s.kind == VDTTFS_LAYER_POOL) {
+            VD_TRY(launch_step_pool(ctx, in, out, l.s.n, l.s.H_in, l.s.W_in, l.s.C_in, net->steps));
+        } else {
+            StepWindows w;
+            for (int s = 0; s < kStepMaxWin; ++s) w.th[s] = w.th_after[s] = NAN;
+            w.out_layer = i == last;
+            for (int t = 0; t < net->steps; ++t) {
+                bool int_ok, fire_ok;
                 float kv, th;
                 if (t1) {
                     // T1S:74-101: integrate every step, fire from t_min on
@@ -158,7 +150,7 @@ int forward_impl(vdttfs_stepnet* net, const float* d_img, int32_t* d_pred) {
                     if (t_min < 0) t_min = 0;
                     kv = expf(-((float)t - l.td_i) / l.tc_i);
                     th = c.vth * expf(-((float)t - l.td_f) / l.tc_f);
-                    int_ok = 1;
+                    int_ok = true;
                     fire_ok = t >= t_min;
                 } else {
                     // T2S:72-107: layer-local integration and firing windows
@@ -169,20 +161,26 @@ int forward_impl(vdttfs_stepnet* net, const float* d_img, int32_t* d_pred) {
                     th = c.vth * expf(-(t_fire - l.td_f) / l.tc_f);
                     int_ok = t_integ >= 0.0f && t_integ < (float)T;
                     fire_ok = t_fire >= start && t_fire < (float)T;
-                    if (!int_ok && !fire_ok && i != last) {
-                        // outside both windows the step only clears the spikes of
-                        // the neurons that have not fired; nothing spikes
-                        VD_HIP(hipMemsetAsync(l.spk, 0, (size_t)l.s.n, ctx->stream));
-                        s_in = l.spk;
-                        continue;
-                    }
                 }
-                const int out_layer = i == last ? (t1 ? 1 : 2) : 0;
-                VD_TRY(launch_step_neuron(ctx, l.s, s_in, l.spk, l.vmem, l.fired, net->out, net->mode, int_ok,
-                                          fire_ok, out_layer, kv, th, t));
+                // the integration window is one run of steps; the fire
+                // window is one too and does not begin before it
+                if (!(fire_ok && th >= 1e-5f)) th = NAN;  // may not fire (T1S:95)
+                if (int_ok) {
+                    if (w.n_int == 0) w.t0 = (float)t;
+                    if (w.n_int < kStepMaxWin) {
+                        w.kv[w.n_int] = kv;
+                        w.th[w.n_int] = th;
+                    }
+                    ++w.n_int;
+                } else if (fire_ok) {
+                    if (w.n_after == 0) w.t_after = (float)t;
+                    if (w.n_after < kStepMaxWin) w.th_after[w.n_after] = th;
+                    ++w.n_after;
+                }
             }
-            s_in = l.spk;
+            VD_TRY(launch_step_layer(ctx, l.s, in, out, net->mode, w));
         }
+        in = out;
     }
     if (d_pred) {
         const StepLayer& o = net->L.back().s;
