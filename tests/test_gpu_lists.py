@@ -90,3 +90,42 @@ def test_culif_engine_lists(gpu_ctx_factory, T, delta, C1, C2, C3, decay, th):
         net.close()
     for i in range(4):
         np.testing.assert_array_equal(got[i].reshape(-1), ref[i].reshape(-1), err_msg=f"layer {i}")
+
+
+@pytest.mark.parametrize("T,delta,K,C_in,C_out,is_fc", [(64, 16, 3, 20, 70, False), (80, 7, 5, 3, 6, False),
+                                                        (255, 256, 1, 130, 33, False), (48, 1, 1, 300, 260, True)])
+def test_any_bucket_contents(gpu_ctx_factory, T, delta, K, C_in, C_out, is_fc):
+    """Buckets a caller may hand over: offsets that run backwards or past the
+    column, times outside the chunk or the window, infinite and NaN, inputs
+    past the width and repeated.  Past 1024 outputs the loop nest over the
+    chunks runs; its first C_out outputs are the reference."""
+    print(f"buckets T={T} delta={delta} K={K} {C_in}->{C_out}", flush=True)
+    WIDE, B, H, W = 1030, 2, 5, 6
+    if is_fc:
+        H = W = 1
+    tc = vdttfs.task2_consts(T=T, delta=delta, tfs=5.0)
+    ctx = gpu_ctx_factory(tc)
+    rng = np.random.default_rng(T)
+    cols, NC = B * H * W, (T + delta - 1) // delta
+    cin = rng.integers(-2, C_in + 3, (cols, C_in)).astype(np.int32)
+    tin = np.sort(rng.random((cols, C_in)) * (T + 12) - 4, axis=1).astype(np.float32)
+    tin[rng.random(tin.shape) < 0.02] = np.inf
+    tin[rng.random(tin.shape) < 0.02] = np.nan
+    tb = np.clip(np.nan_to_num(tin - 5.0, nan=0.0, posinf=1e6), 0, T).astype(int)
+    off = np.stack([(tb < delta * i).sum(1) for i in range(NC + 1)], axis=1).astype(np.int32)
+    wild = rng.random(off.shape) < 0.1
+    off[wild] += rng.integers(-C_in, C_in, int(wild.sum())).astype(np.int32)
+    Wt = (rng.standard_normal((K * K * C_in, WIDE)) * np.sqrt(2.0 / (K * K * C_in))).astype(np.float32)
+    bias = (rng.standard_normal(WIDE) * 0.2).astype(np.float32)
+    alpha, theta = vdttfs.build_luts_host(tc, 0.75 * T, 0.5, 1.5 * T, 2.5)
+    d = [ctx.to_device(x) for x in (cin.reshape(-1), tin.reshape(-1), off.reshape(-1), alpha, theta)]
+    outs = []
+    for co in (WIDE, C_out):
+        k, b = ctx.to_device(np.ascontiguousarray(Wt[:, :co])), ctx.to_device(bias[:co].copy())
+        o = ctx.empty(cols * co).fill(0xFF)
+        ctx.integrate(o, d[0], d[1], d[2], k, b, d[3], d[4], 2, B=B, H_in=H, W_in=W, C_in=C_in, H_out=H, W_out=W,
+                      C_out=co, K_h=K, K_w=K, is_fc=is_fc)
+        ctx.synchronize()
+        outs.append(o.download().reshape(cols, co))
+    assert (outs[1] < INF).any() and (outs[1] == INF).any()
+    np.testing.assert_array_equal(outs[1], outs[0][:, :C_out])

@@ -49,6 +49,48 @@ struct LateThr {
     int lo, hi, mono;
 };
 
+// A workgroup of 256 threads fills *thr.
+__device__ inline void prepare_thresholds(const float* theta, int T, int t_min, LateThr* thr) {
+    const int lane = lane_id();
+            __shared__ float ths[kSplitMaxT + 1];
+            for (int t = threadIdx.x; t <= kSplitMaxT; t += 256) {
+                const float th = theta && t < T ? theta[t] : 0.0f;
+                ths[t] = (t < T && t >= t_min && th >= 1e-5f) ? th : __builtin_nanf("");
+                if (t < kSplitMaxT) thr->th[t] = ths[t];
+            }
+            __syncthreads();
+            if (threadIdx.x < 64) {
+                int lo = kSplitMaxT, hi = 0;
+    #pragma unroll
+                for (int k = 0; k < kSplitMaxT / 64; ++k) {
+                    const float x = ths[64 * k + lane];
+                    const uint64_t v = __ballot(x == x);
+                    if (v != 0) {
+                        const int f = 64 * k + __ffsll((unsigned long long)v) - 1;
+                        lo = f < lo ? f : lo;
+                        hi = 64 * k + 64 - __clzll((long long)v);
+                    }
+                }
+                lo = lo < hi ? lo : hi;
+                // every step within [lo, hi) down or level (a NaN inside fails)
+                bool down = true;
+    #pragma unroll
+                for (int k = 0; k < kSplitMaxT / 64; ++k) {
+                    const int t = 64 * k + lane;
+                    if (t >= lo && t < hi - 1) down = down && ths[t] >= ths[t + 1];
+                }
+                const bool mono = __ballot(!down) == 0;
+                if (lane == 0) {
+                    const float l0 = hi > lo ? log2f(ths[lo]) : 0.0f, l1 = hi > lo ? log2f(ths[hi - 1]) : 0.0f;
+                    thr->lg0 = l0;
+                    thr->inv = l0 > l1 ? (float)(hi - 1 - lo) / (l0 - l1) : 0.0f;
+                    thr->lo = lo;
+                    thr->hi = hi;
+                    thr->mono = mono;
+                }
+            }
+}
+
 struct SplitArgs {
     const float* in;     // [cols][C_in] spike times
     float* a0;           // null: no bin-0 factors, and the lists hold bin 0's events too; else [cols][Cp] bin-0 factors, C_in padded with zeros to whole groups of 4 HL; element
@@ -80,45 +122,7 @@ __global__ __launch_bounds__(256) void k_split(SplitArgs a, int seg) {
     __shared__ float lut[kSplitMaxT + 1];
     for (int i = threadIdx.x; i <= a.T; i += 256) lut[i] = a.alpha[i];
     const int lane = lane_id(), wave = uniform(threadIdx.x >> 6);
-    if (blockIdx.x == 0) {
-        __shared__ float ths[kSplitMaxT + 1];
-        for (int t = threadIdx.x; t <= kSplitMaxT; t += 256) {
-            const float th = a.theta && t < a.T ? a.theta[t] : 0.0f;
-            ths[t] = (t < a.T && t >= a.t_min && th >= 1e-5f) ? th : __builtin_nanf("");
-            if (t < kSplitMaxT) a.thr->th[t] = ths[t];
-        }
-        __syncthreads();
-        if (threadIdx.x < 64) {
-            int lo = kSplitMaxT, hi = 0;
-#pragma unroll
-            for (int k = 0; k < kSplitMaxT / 64; ++k) {
-                const float x = ths[64 * k + lane];
-                const uint64_t v = __ballot(x == x);
-                if (v != 0) {
-                    const int f = 64 * k + __ffsll((unsigned long long)v) - 1;
-                    lo = f < lo ? f : lo;
-                    hi = 64 * k + 64 - __clzll((long long)v);
-                }
-            }
-            lo = lo < hi ? lo : hi;
-            // every step within [lo, hi) down or level (a NaN inside fails)
-            bool down = true;
-#pragma unroll
-            for (int k = 0; k < kSplitMaxT / 64; ++k) {
-                const int t = 64 * k + lane;
-                if (t >= lo && t < hi - 1) down = down && ths[t] >= ths[t + 1];
-            }
-            const bool mono = __ballot(!down) == 0;
-            if (lane == 0) {
-                const float l0 = hi > lo ? log2f(ths[lo]) : 0.0f, l1 = hi > lo ? log2f(ths[hi - 1]) : 0.0f;
-                a.thr->lg0 = l0;
-                a.thr->inv = l0 > l1 ? (float)(hi - 1 - lo) / (l0 - l1) : 0.0f;
-                a.thr->lo = lo;
-                a.thr->hi = hi;
-                a.thr->mono = mono;
-            }
-        }
-    }
+    if (blockIdx.x == 0) prepare_thresholds(a.theta, a.T, a.t_min, a.thr);
     __syncthreads();
     const int S = 1 << seg, P = 64 >> seg;
     const int sub = lane >> seg, r = lane & (S - 1);
@@ -144,6 +148,77 @@ __global__ __launch_bounds__(256) void k_split(SplitArgs a, int seg) {
             base += __popcll(m);
         }
         if (cok && r == 0) a.cnt[col] = base;
+    }
+}
+
+// The lists of k_late from the reference's buckets: per column the events of
+// its bucket entries in entry order.  An entry counts where the loop nest over
+// the chunks (k_integrate_generic) would take it: its own chunk's offsets,
+// clamped to the column, hold its position, and its step and input are in
+// range.  A step's events all come from one chunk, so entry order is that
+// loop's order within every step.
+struct RefListArgs {
+    const int32_t* cin;  // [cols][C_in]
+    const float* tin;
+    const int32_t* off;  // [cols][n_chunks + 1]
+    int2* late;
+    int32_t* cnt;
+    const float* alpha;
+    const float* theta;
+    LateThr* thr;
+    int64_t cols;
+    int C_in, T, D, alpha_by_time, t_min;
+    float tfs;
+};
+
+__global__ __launch_bounds__(256) void k_ref_lists(RefListArgs a) {
+    const int lane = lane_id(), wave = uniform(threadIdx.x >> 6);
+    if (blockIdx.x == 0) prepare_thresholds(a.theta, a.T, a.t_min, a.thr);
+    const int NC = (a.T + a.D - 1) / a.D;
+    const uint64_t lt = lanemask_lt();
+    for (int64_t col = (int64_t)blockIdx.x * 4 + wave; col < a.cols; col += (int64_t)gridDim.x * 4) {
+        const int32_t* const off = a.off + col * (NC + 1);
+        auto clamped = [&](int c, int* s, int* e) {
+            const int s0 = off[c], e0 = off[c + 1];
+            *s = s0 < 0 ? 0 : (s0 > a.C_in ? a.C_in : s0);
+            *e = e0 < *s ? *s : (e0 > a.C_in ? a.C_in : e0);
+        };
+        // entries past every chunk's end are not read
+        int last = 0;
+        for (int c = lane; c < NC; c += 64) {
+            int s, e;
+            clamped(c, &s, &e);
+            last = e > s && e > last ? e : last;
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            const int x = __shfl_xor(last, o, 64);
+            last = x > last ? x : last;
+        }
+        int base = 0;
+        for (int p0 = 0; p0 < last; p0 += 64) {
+            const int p = p0 + lane;
+            bool ev = p < last;
+            int ci = 0, tb = 0;
+            float t = 0.0f;
+            if (ev) {
+                ci = a.cin[col * a.C_in + p];
+                t = a.tin[col * a.C_in + p];
+                tb = (int)floorf(t - a.tfs);
+                if (tb < 0) tb = 0;
+                ev = tb < a.T && (unsigned)ci < (unsigned)a.C_in;
+            }
+            if (ev) {
+                int s, e;
+                clamped(tb / a.D, &s, &e);
+                ev = p >= s && p < e;
+            }
+            const uint64_t m = __ballot(ev);
+            if (ev)
+                a.late[col * a.C_in + base + __popcll(m & lt)] =
+                    make_int2(ci | (tb << 16), __float_as_int(a.alpha[alpha_index(t, tb, a.alpha_by_time, a.T)]));
+            base += __popcll(m);
+        }
+        if (lane == 0) a.cnt[col] = base;
     }
 }
 
@@ -947,6 +1022,21 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
     return K * pix * s.C_out >= 100000000 || (K >= 1024 && s.C_out > 64);
 }
 
+namespace {
+
+// Sizes k_late takes every bin of.
+bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
+    const int T = ctx->c.T;
+    const int taps = s.is_fc ? 1 : s.K_h * s.K_w;
+    const int64_t cols = split_cols(s), pix = split_pix(s), K = (int64_t)taps * s.C_in;
+    if (T > kSplitMaxT || taps > kSplitMaxTaps || s.C_out > 1024) return false;
+    if (K > 0xFFFF || K * s.C_out * 4 >= kOob) return false;
+    if (cols * s.C_in * 4 >= kOob || pix * 8 >= (INT64_C(1) << 31)) return false;
+    return true;
+}
+
+}  // namespace
+
 // Layers the list form takes (k_split's lists with bin 0's events, then k_late
 // over every bin) in place of bucketize or dense merge, k_merge and k_stream:
 // windows past 64 steps, whose bins the fused kernels' lanes do not hold.
@@ -957,15 +1047,9 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
 // 51.  Each group of four c_out blocks rebuilds a pixel's list and below 32
 // c_out a wave is mostly idle, so wide layers and narrow convolutions keep the
 // merged lists.
-bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
-    const int T = ctx->c.T;
-    const int taps = s.is_fc ? 1 : s.K_h * s.K_w;
-    const int64_t cols = split_cols(s), pix = split_pix(s), K = (int64_t)taps * s.C_in;
-    if (T > kSplitMaxT || taps > kSplitMaxTaps || s.C_out > 1024 || (s.C_out < 32 && !s.is_fc)) return false;
-    if (K > 0xFFFF || K * s.C_out * 4 >= kOob) return false;
-    if (cols * s.C_in * 4 >= kOob || pix * 8 >= (INT64_C(1) << 31)) return false;
-    return T > 64;
-}
+bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64 && (s.C_out >= 32 || s.is_fc) && lists_fit(ctx, s); }
+
+bool ref_lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return lists_fit(ctx, s); }
 
 namespace {
 
@@ -975,6 +1059,15 @@ struct LateScratch {
     int32_t* cnt;
     LateThr* thr;
 };
+
+void carve(void* scratch, int64_t cols, int C_in, LateScratch* sc) {
+    unsigned char* sp = static_cast<unsigned char*>(scratch);
+    sc->late = reinterpret_cast<int2*>(sp);
+    sp += align256((size_t)cols * C_in * 8);
+    sc->cnt = reinterpret_cast<int32_t*>(sp);
+    sp += align256((size_t)cols * 4);
+    sc->thr = reinterpret_cast<LateThr*>(sp);
+}
 
 template <LateMode MODE>
 int launch_late(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const LateScratch& sc, const float* W,
@@ -1082,18 +1175,29 @@ int launch_split(vdttfs_ctx* ctx, const SplitArgs& k) {
 
 }  // namespace
 
+int launch_integrate_ref_lists(vdttfs_ctx* ctx, float* out, const int32_t* cin, const float* tin, const int32_t* off,
+                               void* scratch, const float* W, const float* bias, const float* alpha,
+                               const float* theta, int t_min, const IntegShape& s) {
+    const int64_t cols = split_cols(s);
+    if (cols == 0 || split_pix(s) == 0) return VDTTFS_OK;
+    LateScratch sc;
+    carve(scratch, cols, s.C_in, &sc);
+    RefListArgs a{cin, tin, off, sc.late, sc.cnt, alpha, theta, sc.thr, cols, s.C_in, ctx->c.T, ctx->c.delta,
+                  ctx->c.alpha_by_time, t_min, ctx->c.tfs};
+    int64_t blocks = (cols + 3) / 4;
+    if (blocks > 8192) blocks = 8192;
+    hipLaunchKernelGGL(k_ref_lists, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a);
+    VD_HIP(hipGetLastError());
+    return launch_late<kLateAll>(ctx, out, nullptr, alpha, sc, W, bias, theta, t_min, s, nullptr);
+}
+
 int launch_integrate_lists(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
                            const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s,
                            const CulifNeuron* culif) {
     const int64_t cols = split_cols(s);
     if (cols == 0 || split_pix(s) == 0) return VDTTFS_OK;
-    unsigned char* sp = static_cast<unsigned char*>(scratch);
     LateScratch sc;
-    sc.late = reinterpret_cast<int2*>(sp);
-    sp += align256((size_t)cols * s.C_in * 8);
-    sc.cnt = reinterpret_cast<int32_t*>(sp);
-    sp += align256((size_t)cols * 4);
-    sc.thr = reinterpret_cast<LateThr*>(sp);
+    carve(scratch, cols, s.C_in, &sc);
     VD_TRY(launch_split(ctx, SplitArgs{in, nullptr, sc.late, sc.cnt, alpha, theta, sc.thr, cols, s.C_in, s.C_in,
                                        ctx->c.T, ctx->c.alpha_by_time, t_min, 1, ctx->c.tfs}));
     if (culif) return launch_late<kLateCulif>(ctx, out, in, alpha, sc, W, bias, theta, t_min, s, culif);
