@@ -24,6 +24,9 @@ SHAPES = [
     ("t255-conv5-32-64", 255, 0, False, False, 3, 9, 8, 32, 64, 5),
     ("t100-conv3-200-70", 100, 0, True, False, 2, 4, 3, 200, 70, 3),
     ("t255-conv3-24-1024", 255, 0, True, False, 1, 3, 3, 24, 1024, 3),
+    ("t80-conv5-1-6", 80, 0, False, False, 3, 28, 28, 1, 6, 5),
+    ("t80-conv5-6-16", 80, 0, False, False, 3, 12, 12, 6, 16, 5),
+    ("t65-conv3-7-31", 65, 0, True, False, 3, 5, 6, 7, 31, 3),
     ("t80-fc-1600-128", 80, 0, True, True, 9, 1, 1, 1600, 128, 1),
     ("t80-fc-128-10", 80, 0, True, True, 17, 1, 1, 128, 10, 1),
     ("t200-fc-4100-700", 200, 0, False, True, 3, 1, 1, 4100, 700, 1),

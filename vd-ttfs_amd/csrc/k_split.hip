@@ -1044,10 +1044,13 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
 // 387 -> 190 us, 128->128 at 16x16: 321 -> 132; LeNet-5's FC layers at T = 80,
 // batch 128: 113 -> 51.  At T = 64 the fused kernels win: CuLIF 64->128 at
 // 128x128 2248 against 2460 us, LeNet-5's FC layers at batch 1024 45 against
-// 51.  Each group of four c_out blocks rebuilds a pixel's list and below 32
-// c_out a wave is mostly idle, so wide layers and narrow convolutions keep the
-// merged lists.
-bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64 && (s.C_out >= 32 || s.is_fc) && lists_fit(ctx, s); }
+// 51.  Layers narrower than a wave leave most of its lanes idle and still win
+// past 64 steps (LeNet-5 at T = 80: conv1, 6 outputs, 32 -> 11 us for one image
+// and 128 -> 78 for 128; conv2, 16 outputs, 37 -> 20 and 48 -> 37); at T = 64
+// the register and narrow kernels do (batch 1024: conv1 145 against 567 us,
+// conv2 169 against 169).  Each group of four c_out blocks rebuilds a pixel's
+// list, so layers past 1024 outputs keep the merged lists.
+bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64 && lists_fit(ctx, s); }
 
 bool ref_lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return lists_fit(ctx, s); }
 
