@@ -193,6 +193,10 @@ int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const f
 // The same lists over every bin, with the LUT or the CuLIF neuron (windows past
 // 64 steps); in split_scratch_bytes of scratch.
 bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s);
+// Small fields and few outputs, one pixel per lane (k_pixel.hip).
+bool conv_px_ok(const IntegShape& s);
+int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W, const float* bias,
+                   const float* theta, int t_min, const IntegShape& s);
 // ... and over the reference's buckets.
 bool ref_lists_ok(const vdttfs_ctx* ctx, const IntegShape& s);
 int launch_integrate_ref_lists(vdttfs_ctx* ctx, float* out, const int32_t* cin, const float* tin, const int32_t* off,

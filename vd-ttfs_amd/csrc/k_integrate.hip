@@ -3845,6 +3845,9 @@ bool small_ok(const vdttfs_ctx* ctx, const IntegShape& sh) {
 
 int launch_conv_small(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W,
                       const float* bias, const float* theta, int t_min, const IntegShape& sh) {
+    // up to 16 outputs a lane holds all of a pixel (LeNet-5's conv1, batch
+    // 1024: 145 -> 34 us); wider layers would leave too few registers
+    if (conv_px_ok(sh)) return launch_conv_px(ctx, out, in, alpha, W, bias, theta, t_min, sh);
     SmallArgs a{};
     a.in = in;
     a.alpha = alpha;
@@ -4001,9 +4004,9 @@ int resolve_named(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan&
         *out = p;
         return VDTTFS_OK;
     }
-    // no list (k_conv_small).  Built-in for layers narrower than 32 outputs
-    // (LeNet conv1, B=1024: 0.37 ms against 0.58 for k_merge_dense +
-    // k_stream_narrow).  A wave-wide layer keeps the fused list: k_conv_small
+    // no list (k_conv_small; up to 16 outputs k_conv_px).  Built-in for layers
+    // narrower than 32 outputs (LeNet conv1, B=1024: k_conv_px 34 us,
+    // k_conv_small 145, k_merge_dense + k_stream_narrow 580).  A wave-wide layer keeps the fused list: k_conv_small
     // scans every element for each occupied bin, about 5,400 instructions
     // per VGG-16 L0 pixel against 2,600 for k_stream_dense (1.42 against
     // 0.70 ms), which touches each event once.

@@ -1045,8 +1045,8 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
 // batch 128: 113 -> 51.  At T = 64 the fused kernels win: CuLIF 64->128 at
 // 128x128 2248 against 2460 us, LeNet-5's FC layers at batch 1024 45 against
 // 51.  Layers narrower than a wave leave most of its lanes idle and still win
-// past 64 steps (LeNet-5 at T = 80: conv1, 6 outputs, 32 -> 11 us for one image
-// and 128 -> 78 for 128; conv2, 16 outputs, 37 -> 20 and 48 -> 37); at T = 64
+// past 64 steps (LeNet-5's conv2 at T = 80, 16 outputs: 37 -> 20 us for one
+// image, 48 -> 37 for 128); at T = 64
 // the register and narrow kernels do (batch 1024: conv1 145 against 567 us,
 // conv2 169 against 169).  Each group of four c_out blocks rebuilds a pixel's
 // list, so layers past 1024 outputs keep the merged lists.
@@ -1199,6 +1199,8 @@ int launch_integrate_lists(vdttfs_ctx* ctx, float* out, const float* in, const f
                            const CulifNeuron* culif) {
     const int64_t cols = split_cols(s);
     if (cols == 0 || split_pix(s) == 0) return VDTTFS_OK;
+    // small fields need no lists (LeNet-5's conv1 at T = 80, batch 128: 78 -> 13 us)
+    if (!culif && conv_px_ok(s)) return launch_conv_px(ctx, out, in, alpha, W, bias, theta, t_min, s);
     LateScratch sc;
     carve(scratch, cols, s.C_in, &sc);
     VD_TRY(launch_split(ctx, SplitArgs{in, nullptr, sc.late, sc.cnt, alpha, theta, sc.thr, cols, s.C_in, s.C_in,
