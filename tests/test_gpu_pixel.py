@@ -1,4 +1,4 @@
-"""Convolutions of small fields and few outputs (one pixel per lane) against
+"""Narrow convolutions (one pixel per lane or per four lanes) against
 the oracle, bit for bit: every field and output width of the kernel, odd ones
 between them, padding, windows of one to four blocks of 64 bins, fire starts,
 thresholds that do not fall, weights that are not finite, partial waves."""
@@ -22,6 +22,12 @@ SHAPES = [
     ("t130-conv5-1-13-same", 130, 7, True, False, 2, 11, 6, 1, 13, 5),
     ("t33-conv3-2-9", 33, 0, False, False, 4, 5, 5, 2, 9, 3),
     ("t64-conv5-1-3-big", 64, 0, False, False, 90, 32, 32, 1, 3, 5),  # 256 threads a workgroup
+    # four lanes a pixel: every width of theirs, odd sizes, padding
+    ("t64-conv3-4-16-same", 64, 0, True, False, 9, 31, 30, 4, 16, 3),
+    ("t80-conv3-7-5", 80, 0, False, False, 11, 30, 29, 7, 5, 3),
+    ("t64-conv3-12-13-same", 64, 9, True, False, 9, 31, 30, 12, 13, 3),
+    ("t64-conv5-6-16", 64, 0, False, False, 90, 31, 32, 6, 16, 5),
+    ("t140-conv1-160-10", 140, 0, True, False, 80, 29, 29, 160, 10, 1),
 ]
 KINDS = ["random", "silent", "bin0", "last-bin", "dense", "fractional"]
 

@@ -316,7 +316,7 @@ int forward_impl(vdttfs_culif_net* net, const float* d_data, int32_t* d_pred, ui
                 // map (the bin-layout bucketize then only counts retained events)
                 LaunchPlan plan;
                 VD_TRY(resolve_plan(ctx, sh, LaunchPlan{}, &plan));
-                if (!count_here && lists_ok(ctx, sh)) {
+                if (!count_here && ctx->c.T > 64 && lists_ok(ctx, sh)) {
                     VD_TRY(launch_integrate_lists(ctx, l.out, cur, net->ones, net->list, l.W, nullptr, nullptr, 0, sh,
                                                   &nrn));
                     break;

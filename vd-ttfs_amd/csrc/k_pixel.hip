@@ -1,28 +1,31 @@
-// Conv layers with a small receptive field (at most 32 elements) and few
-// outputs (at most 16): one pixel per lane, all its outputs in registers
-// (LeNet-5's conv1, T1V:83-162).
+// Narrow conv layers (at most 16 outputs) with at most 160 elements in a field:
+// one pixel per lane, or per four lanes, with all its outputs in registers
+// (LeNet-5's convolutions, T1V:83-162).
 //
-// A lane loads its pixel's field and packs every event into one key, {bin,
-// element, decay index}, so that the smallest key above the last one is the
-// next event in the reference's order: bins ascending, within a bin (kh, kw,
-// cin).  Finding it takes a subtract per element and a three-way minimum per
-// two; the event then adds its weight row (LDS) to the open bin's sums of all
-// outputs.  Where a bin closes, the carry stands until the lane's next event,
-// and with thresholds that fall over the window a neuron fires in that run
-// iff its carry reaches the run's last threshold; the step itself is searched
-// once per neuron at the end.
+// A lane loads its elements of the field and packs every event into one key,
+// {bin, element, decay index}, so that the smallest key above the last one is
+// the next event in the reference's order: bins ascending, within a bin (kh,
+// kw, cin).  Finding it takes a subtract per element and a three-way minimum
+// per two; the event then adds its weight row (LDS) to the open bin's sums of
+// all outputs.  Where a bin closes, the carry stands until the pixel's next
+// event, and with thresholds that fall over the window a neuron fires in that
+// run iff its carry reaches the run's last threshold; the step itself is
+// searched once per neuron at the end.
 //
-// Bound by instruction issue: about 40 instructions per event and pixel for
-// the search and 12 per output.  The register kernel it stands in for
-// (k_conv_small, one output per lane) compares every element with every
-// occupied bin, 75 instructions per bin for ten pixels of LeNet-5's conv1.
+// Bound by instruction issue: 1.5 instructions per element and event for the
+// search and about 12 per output.  Up to 32 elements a lane has a pixel to
+// itself (25 elements, 6 outputs, 590K pixels, T = 64: 34 us; one output per
+// lane, every element compared with every occupied bin, took 145).  Past that
+// four lanes share the elements and the outputs of a pixel: a lane alone needs
+// all registers and leaves one wave per SIMD (150 elements, 16 outputs, 66K
+// pixels: 160 us against 136; eight lanes 163).
 #include "common.h"
 #include "wave.h"
 
 namespace vdttfs {
 namespace {
 
-constexpr int kPxMaxEl = 32;
+constexpr int kPxMaxEl = 160;  // a key holds an element in 8 bits
 constexpr int kPxMaxOut = 16;
 
 struct PxArgs {
@@ -43,11 +46,21 @@ struct PxArgs {
     int dk[kPxMaxEl], tap[kPxMaxEl];
 };
 
-template <int CO, int NEL>
+// The smallest value of a group of G lanes.
+template <int G>
+__device__ __forceinline__ unsigned group_min(unsigned v) {
+    auto with = [&](unsigned x) { v = x < v ? x : v; };
+    if constexpr (G > 1) with((unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));  // lane ^ 1
+    if constexpr (G > 2) with((unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));  // lane ^ 2
+    return v;
+}
+
+// G lanes share a pixel: each holds CO outputs and NEL elements, e = G i + g.
+template <int G, int CO, int NEL>
 __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
-    constexpr int COP = (CO + 3) & ~3;
+    constexpr int COP = G * ((CO + 3) & ~3);
     constexpr unsigned kNone = ~0u;
-    __shared__ __attribute__((aligned(16))) float w_lds[NEL * COP];
+    __shared__ __attribute__((aligned(16))) float w_lds[G * NEL * COP];
     __shared__ float lut[256], th[256];  // th: the threshold where a spike may occur, else NaN
     const int T = a.T;
     for (int i = threadIdx.x; i < a.nel * COP; i += blockDim.x) {
@@ -60,7 +73,8 @@ __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
         th[t] = (t < T && t >= a.t_min && x >= 1e-5f) ? x : __builtin_nanf("");
     }
     // the lane's field
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    const int g = threadIdx.x & (G - 1), c0 = g * CO;
+    const int idx = (blockIdx.x * blockDim.x + threadIdx.x) / G;
     const bool ok = idx < a.n_pix;
     const int px = ok ? idx : a.n_pix - 1;
     const int qd = fdiv(px, a.div_w);
@@ -71,7 +85,18 @@ __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
     const __amdgpu_buffer_rsrc_t rin =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.in, (short)0, a.in_bytes, 0x00020000);
     float time[NEL];
-    if (a.inside) {  // uniform
+    if constexpr (G > 1) {
+#pragma unroll
+        for (int i = 0; i < NEL; ++i) {
+            const int e = G * i + g < a.nel ? G * i + g : 0;
+            const int tap = a.tap[e];
+            const bool inb = (unsigned)(h0 + (tap >> 16)) < (unsigned)a.H_in &&
+                             (unsigned)(w0 + (tap & 0xFFFF)) < (unsigned)a.W_in;
+            const float t =
+                __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rin, inb ? (base + a.dk[e]) * 4 : 0, 0, 0));
+            time[i] = inb ? t : kInfTime;
+        }
+    } else if (a.inside) {  // uniform
 #pragma unroll
         for (int e = 0; e < NEL; ++e)  // past nel: element 0 (dk 0)
             time[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rin, base * 4, a.dk[e] * 4, 0));
@@ -108,19 +133,20 @@ __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
     // alpha_index without branches)
     unsigned key[NEL];
 #pragma unroll
-    for (int e = 0; e < NEL; ++e) {
-        const float t = time[e];
+    for (int i = 0; i < NEL; ++i) {
+        const int e = G * i + g;
+        const float t = time[i];
         const int tb = (int)floorf(fmaxf(t - a.tfs, 0.0f));
         const bool ev = e < a.nel && t < kInfTime && tb < T;
         const int ai = a.alpha_by_time ? (int)__builtin_amdgcn_fmed3f(t, 0.0f, (float)T) : tb;
-        key[e] = ev ? (unsigned)(tb << 16 | e << 8 | ai) : kNone;
+        key[i] = ev ? (unsigned)(tb << 16 | e << 8 | ai) : kNone;
     }
     float acc[CO], carry[CO], at_fire[CO];
     int from[CO];  // a neuron that fires: its run's first bin that may (its step, where not mono), else -1
 #pragma unroll
     for (int c = 0; c < CO; ++c) {
         acc[c] = 0.0f;
-        carry[c] = c < a.C_out ? a.bias[c] : 0.0f;
+        carry[c] = c0 + c < a.C_out ? a.bias[c0 + c] : 0.0f;
         at_fire[c] = 0.0f;
         from[c] = -1;
     }
@@ -153,14 +179,15 @@ __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
     unsigned m = key[0];
 #pragma unroll
     for (int e = 1; e < NEL; ++e) m = key[e] < m ? key[e] : m;
+    m = group_min<G>(m);
     test(0, m == kNone ? T : (int)(m >> 16));
     while (m != kNone) {
         const int b = (int)(m >> 16);
         const float al = lut[m & 0xFF];
-        const float* const w = w_lds + ((m >> 8) & 0xFF) * COP;
-        float wv[COP];
+        const float* const w = w_lds + ((m >> 8) & 0xFF) * COP + c0;
+        float wv[(CO + 3) & ~3];
 #pragma unroll
-        for (int c = 0; c < COP; c += 4) *reinterpret_cast<float4*>(wv + c) = *reinterpret_cast<const float4*>(w + c);
+        for (int c = 0; c < CO; c += 4) *reinterpret_cast<float4*>(wv + c) = *reinterpret_cast<const float4*>(w + c);
 #pragma unroll
         for (int c = 0; c < CO; ++c) acc[c] = __builtin_fmaf(wv[c], al, acc[c]);
         // the smallest key above m: those at or below it, and kNone, stay past
@@ -172,6 +199,7 @@ __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
             const unsigned x = key[e] - m1;
             d = x < d ? x : d;
         }
+        d = group_min<G>(d);
         m = d < (1u << 24) ? d + m1 : kNone;
         const int b2 = m == kNone ? T : (int)(m >> 16);
         if (b2 != b) {
@@ -207,15 +235,22 @@ __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
     }
 #pragma unroll
     for (int c = 0; c < CO; ++c)
-        if (c < a.C_out) po[c] = from[c] < 0 ? kInfTime : (float)from[c];
+        if (c0 + c < a.C_out) po[c0 + c] = from[c] < 0 ? kInfTime : (float)from[c];
 }
 
 }  // namespace
 
+// Past 32 elements the search costs more than a list, which finds its order
+// once, unless the pixels fill the chip: k_merge_dense + k_stream_narrow
+// against this, T = 64: 108 elements, 16K pixels 50 -> 39 us (density 0.5) and
+// 40 -> 23 (0.1); 150 elements, 66K pixels 168 -> 136, but 33K pixels 95 ->
+// 120.
 bool conv_px_ok(const IntegShape& s) {
     const int64_t in = (int64_t)s.B * s.H_in * s.W_in * s.C_in * 4, pix = (int64_t)s.B * s.H_out * s.W_out;
-    return !s.is_fc && (int64_t)s.K_h * s.K_w * s.C_in <= kPxMaxEl && s.C_out <= kPxMaxOut &&
-           in < (INT64_C(1) << 31) && pix < (INT64_C(1) << 31) - 256;
+    const int64_t nel = (int64_t)s.K_h * s.K_w * s.C_in;
+    if (s.is_fc || s.C_out > kPxMaxOut || nel > kPxMaxEl) return false;
+    if (in >= (INT64_C(1) << 31) || 4 * pix >= (INT64_C(1) << 31) - 256) return false;
+    return nel <= 32 || pix >= (nel <= 112 ? 8192 : 65536);
 }
 
 int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W, const float* bias,
@@ -255,20 +290,28 @@ int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* al
             }
     // few pixels: one wave per workgroup, so that they spread over the CUs
     const int threads = a.n_pix >= 256 * 256 ? 256 : 64;
-    const dim3 grid((unsigned)((a.n_pix + threads - 1) / threads)), block(threads);
-#define VD_PX(C, N) hipLaunchKernelGGL((k_conv_px<C, N>), grid, block, 0, ctx->stream, a)
-#define VD_PX_N(C)         \
-    do {                   \
-        if (a.nel <= 9)    \
-            VD_PX(C, 9);   \
+    const int G = a.nel > 32 ? 4 : 1;
+    const dim3 grid((unsigned)(((int64_t)a.n_pix * G + threads - 1) / threads)), block(threads);
+#define VD_PX(G_, C, N) hipLaunchKernelGGL((k_conv_px<G_, C, N>), grid, block, 0, ctx->stream, a)
+#define VD_PX_N(C)            \
+    do {                      \
+        if (a.nel <= 9)       \
+            VD_PX(1, C, 9);   \
         else if (a.nel <= 16) \
-            VD_PX(C, 16);  \
+            VD_PX(1, C, 16);  \
         else if (a.nel <= 25) \
-            VD_PX(C, 25);  \
-        else               \
-            VD_PX(C, 32);  \
+            VD_PX(1, C, 25);  \
+        else                  \
+            VD_PX(1, C, 32);  \
     } while (0)
-    if (a.C_out <= 4)
+    if (G > 1) {
+        if (a.nel <= 64)
+            VD_PX(4, 4, 16);
+        else if (a.nel <= 112)
+            VD_PX(4, 4, 28);
+        else
+            VD_PX(4, 4, 40);
+    } else if (a.C_out <= 4)
         VD_PX_N(4);
     else if (a.C_out <= 6)
         VD_PX_N(6);

@@ -1050,7 +1050,11 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
 // the register and narrow kernels do (batch 1024: conv1 145 against 567 us,
 // conv2 169 against 169).  Each group of four c_out blocks rebuilds a pixel's
 // list, so layers past 1024 outputs keep the merged lists.
-bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64 && lists_fit(ctx, s); }
+bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
+    // (fields past 32 elements that go without lists; smaller ones have a plan)
+    const bool px = conv_px_ok(s) && s.K_h * s.K_w * s.C_in > 32;
+    return (ctx->c.T > 64 || px) && lists_fit(ctx, s);
+}
 
 bool ref_lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return lists_fit(ctx, s); }
 
@@ -1199,7 +1203,7 @@ int launch_integrate_lists(vdttfs_ctx* ctx, float* out, const float* in, const f
                            const CulifNeuron* culif) {
     const int64_t cols = split_cols(s);
     if (cols == 0 || split_pix(s) == 0) return VDTTFS_OK;
-    // small fields need no lists (LeNet-5's conv1 at T = 80, batch 128: 78 -> 13 us)
+    // small fields go without lists (LeNet-5's conv1 at T = 80, batch 128: 78 -> 13 us)
     if (!culif && conv_px_ok(s)) return launch_conv_px(ctx, out, in, alpha, W, bias, theta, t_min, s);
     LateScratch sc;
     carve(scratch, cols, s.C_in, &sc);
