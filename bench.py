@@ -551,8 +551,9 @@ def bench_ttfs(args) -> int:
                       "other conv with <= 9 taps and FC layer whose pixel takes at most two workgroups: 64 or 128 "
                       "c_out per wave, c_out groups pinned to XCDs); otherwise k_merge_dense + k_stream_lean or "
                       "k_bucketize + k_merge + k_stream_lean (e.g. config 5's 4096-wide FC); layers with C_out < "
-                      "32 stream with k_stream_narrow, or with k_conv_small when the receptive field has <= 32 "
-                      "elements.  A launch is one layer's integrate; achieved = rocprofv3 FETCH_SIZE + WRITE_SIZE "
+                      "32 stream with k_stream_narrow, with k_conv_small when the receptive field has <= 32 "
+                      "elements, or with k_conv_px up to 16 c_out; layers whose fire start is a quarter of the "
+                      "window or more (VGG-16) take k_split + k_gemm0 (bin 0 on the matrix cores) + k_late.  A launch is one layer's integrate; achieved = rocprofv3 FETCH_SIZE + WRITE_SIZE "
                       "bytes of the integrator dispatches of one forward / the live HIP-event integrator time of "
                       "a forward",
             "traffic_per_step": tr["per_step"] if tr else None,

@@ -35,9 +35,10 @@ import re
 import sys
 
 # every kernel of a layer's integrate: bucketize (FC layers), merge, stream
-INTEGRATOR = ("k_bucketize", "k_merge", "k_stream", "k_integrate_generic", "k_conv_small")
+INTEGRATOR = ("k_bucketize", "k_merge", "k_stream", "k_integrate_generic", "k_conv_small", "k_conv_px", "k_split",
+              "k_gemm0", "k_late")
 # the dispatch that ends a layer's integrate (lists, if any, come before it)
-LAYER_END = ("k_stream", "k_integrate_generic", "k_conv_small")
+LAYER_END = ("k_stream", "k_integrate_generic", "k_conv_small", "k_conv_px", "k_late")
 COPY_BYTES_DEFAULT = 1 << 30  # bench.py --copy-calibration moves 2^28 floats each way
 
 
