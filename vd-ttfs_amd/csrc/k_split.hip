@@ -983,6 +983,12 @@ size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
 
 }  // namespace
 
+// k_late's grid: a wave per pixel and 64 outputs, up to three idle ones in a
+// group; a launch holds below 2^32 threads.
+static bool late_grid_ok(int64_t pix, int C_out) {
+    return pix < (INT64_C(1) << 31) - 1024 && pix * 64 * ((C_out + 63) / 64 + 3) < (INT64_C(1) << 32);
+}
+
 size_t split_scratch_bytes(const IntegShape& s) {
     const size_t cols = (size_t)split_cols(s);
     return align256(cols * ceil16(s.C_in) * 4) + align256(cols * s.C_in * 8) + align256(cols * 4) +
@@ -997,7 +1003,7 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
     // 16-bit weight rows in a list entry, row 0xFFFF past the weights; 32-bit buffer offsets
     if (K > 0xFFFF || K * s.C_out * 4 >= kOob) return false;
     if (cols * ceil16(s.C_in) * 4 >= kOob) return false;
-    if (pix * ((s.C_out + 63) / 64) >= (INT64_C(1) << 31) - 1024) return false;  // pixels and grids in 31 bits
+    if (!late_grid_ok(pix, s.C_out)) return false;
     // Bin 0 collects the spikes up to the fire start: from a quarter of the
     // window on it holds enough of them that the dense sum beats the gather
     // (VGG-16's layers hold 70-85% there at half the window; layers with a
@@ -1031,8 +1037,7 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
     const int64_t cols = split_cols(s), pix = split_pix(s), K = (int64_t)taps * s.C_in;
     if (T > kSplitMaxT || taps > kSplitMaxTaps || s.C_out > 1024) return false;
     if (K > 0xFFFF || K * s.C_out * 4 >= kOob) return false;
-    if (cols * s.C_in * 4 >= kOob || pix * 8 >= (INT64_C(1) << 31)) return false;
-    return true;
+    return cols * s.C_in * 4 < kOob && late_grid_ok(pix, s.C_out);
 }
 
 }  // namespace

@@ -39,7 +39,7 @@ struct StepArgs {
     float* out;        // first-spike steps, else +inf (T1S output: 9999); T2S output layer: max(V + b)
     const float* W;
     const float* bias;
-    int64_t n;
+    int64_t n, n0;     // neurons, and the first of this launch
     int H_in, W_in, C_in, H_out, W_out, C_out, K_h, K_w, pad_h, pad_w;
     StepWindows w;
 };
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(64) void k_step_layer(StepArgs a) {
     float kvr[kStepMaxWin / 64];  // T2S: kv of step 64 k + lane
 #pragma unroll
     for (int k = 0; k < kStepMaxWin / 64; ++k) kvr[k] = MODE == 2 ? a.w.kv[64 * k + lane] : 0.0f;
-    const int64_t nid_raw = (int64_t)blockIdx.x * 64 + lane;
+    const int64_t nid_raw = a.n0 + (int64_t)blockIdx.x * 64 + lane;
     const bool real = nid_raw < a.n;
     const int64_t nid = real ? nid_raw : a.n - 1;
     const int64_t q = nid / a.C_out;
@@ -184,7 +184,7 @@ unsigned step_grid(int64_t n) {
 
 int launch_step_layer(vdttfs_ctx* ctx, const StepLayer& L, const float* in, float* out, int mode,
                       const StepWindows& w) {
-    if (L.n == 0) return VDTTFS_OK;
+    if (L.n <= 0) return VDTTFS_OK;
     if (w.n_int < 0 || w.n_int > kStepMaxWin || w.n_after < 0 || w.n_after > kStepMaxWin)
         return set_error(VDTTFS_E_UNSUPPORTED, "step layer: windows of %d and %d steps", w.n_int, w.n_after);
     StepArgs a{};
@@ -204,19 +204,22 @@ int launch_step_layer(vdttfs_ctx* ctx, const StepLayer& L, const float* in, floa
     a.pad_h = L.is_fc ? 0 : L.pad_h;
     a.pad_w = L.is_fc ? 0 : L.pad_w;
     a.w = w;
-    const int64_t blocks = (L.n + 63) / 64;
-    if (blocks > 0x7fffffff) return set_error(VDTTFS_E_UNSUPPORTED, "step layer: grid too large");
     const size_t lds = (size_t)64 * ((w.n_int + 7) & ~7) * 4;
     const bool pad = a.pad_h != 0 || a.pad_w != 0;
-    if (mode == 1 && pad)
-        hipLaunchKernelGGL((k_step_layer<1, true>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
-    else if (mode == 1)
-        hipLaunchKernelGGL((k_step_layer<1, false>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
-    else if (pad)
-        hipLaunchKernelGGL((k_step_layer<2, true>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
-    else
-        hipLaunchKernelGGL((k_step_layer<2, false>), dim3((unsigned)blocks), dim3(64), lds, ctx->stream, a);
-    VD_HIP(hipGetLastError());
+    constexpr int64_t kMost = INT64_C(1) << 30;  // a launch's neurons: a grid holds below 2^32 threads
+    for (a.n0 = 0; a.n0 < L.n; a.n0 += kMost) {
+        const int64_t left = L.n - a.n0;
+        const dim3 blocks((unsigned)(((left < kMost ? left : kMost) + 63) / 64));
+        if (mode == 1 && pad)
+            hipLaunchKernelGGL((k_step_layer<1, true>), blocks, dim3(64), lds, ctx->stream, a);
+        else if (mode == 1)
+            hipLaunchKernelGGL((k_step_layer<1, false>), blocks, dim3(64), lds, ctx->stream, a);
+        else if (pad)
+            hipLaunchKernelGGL((k_step_layer<2, true>), blocks, dim3(64), lds, ctx->stream, a);
+        else
+            hipLaunchKernelGGL((k_step_layer<2, false>), blocks, dim3(64), lds, ctx->stream, a);
+        VD_HIP(hipGetLastError());
+    }
     return VDTTFS_OK;
 }
 
