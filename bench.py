@@ -71,7 +71,8 @@ HBM_PEAK_GBS = 8000.0
 COPY_FLOATS = 1 << 28  # 1 GiB read + 1 GiB written per calibration dispatch
 CSRC = os.path.join(ROOT, "vd-ttfs_amd", "csrc")
 # the sources that decide the integrator's dispatches and their memory traffic
-INTEG_SOURCES = ("k_integrate.hip", "k_bucketize.hip", "net.cpp", "capi.cpp", "k_culif.hip", "culif.cpp", "wave.h")
+INTEG_SOURCES = ("k_integrate.hip", "k_split.hip", "k_pixel.hip", "k_bucketize.hip", "net.cpp", "capi.cpp",
+                 "k_culif.hip", "culif.cpp", "wave.h")
 # gather-roof probe: rows uniformly random over a footprint that fits one XCD's 4 MB L2
 PROBE_L2_BYTES = 2 << 20
 PROBE_WAVES, PROBE_EVENTS, PROBE_REPS = 32768, 512, 5
