@@ -2,6 +2,8 @@
 the oracle, bit for bit: every field and output width of the kernel, odd ones
 between them, padding, windows of one to four blocks of 64 bins, fire starts,
 thresholds that do not fall, weights that are not finite, partial waves."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -66,3 +68,27 @@ def test_pixel_odd_tables_and_weights(gpu_ctx_factory, shape, what):
     ref = reference(shape, tc, ho, wo, Wt, bias, sp, alpha, theta, 2)
     got = run(gpu_ctx_factory(tc), shape, ho, wo, Wt, bias, sp, alpha, theta, 2)
     np.testing.assert_array_equal(got, ref, err_msg=f"{shape[0]} {what}")
+
+
+@pytest.mark.parametrize("T", [64, 80])
+def test_pixel_layers_allocate_nothing(gpu_ctx_factory, T):
+    """LeNet-5's conv2 at batch 1024 runs without lists, which would take 90 MB."""
+    print(f"pixel scratch T={T}", flush=True)
+    ctx = gpu_ctx_factory(vdttfs.task1_consts(T=T, delta=16))
+    B, H, C_in, C_out, K = 1024, 12, 6, 16, 5
+    rng = np.random.default_rng(T)
+    sp = np.where(rng.random(B * H * H * C_in) < 0.3, np.floor(rng.random(B * H * H * C_in) * T), INF)
+    alpha, theta = vdttfs.build_luts_host(vdttfs.task1_consts(T=T, delta=16), 16.0, 0.0, 16.0, 0.0)
+    d = [ctx.to_device(v.astype(np.float32)) for v in (sp, rng.standard_normal((150, C_out)) * 0.1, np.zeros(C_out),
+                                                       alpha, theta)]
+    out = ctx.empty(B * 8 * 8 * C_out)
+
+    def free_bytes():
+        ctx.synchronize()
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert ctypes.CDLL("libamdhip64.so").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    before = free_bytes()
+    ctx.layer_forward(out, *d, 0, B, H, H, C_in, 8, 8, C_out, K, K, False)
+    assert before - free_bytes() < 16 << 20  # a kernel's first launch may load its code

@@ -367,6 +367,8 @@ static int engine_layer(vdttfs_ctx* ctx, float* d_out, const float* d_in, const 
     const int64_t cap = merged_list_cap(s);
     const bool dense = plan_from_dense(ctx, s, p, counters != nullptr);
     const bool lds_list = plan_lds_list(ctx, s, p, counters != nullptr, false);
+    if (p.split == kSplitPixel && !counters)  // no scratch
+        return launch_conv_px(ctx, d_out, d_in, d_lut_decay, d_kernel, d_bias, d_lut_th, t_min, s);
     if (p.split && !counters) {
         // as much as the named plan would take, so that a counting call of the
         // layer finds its lists' scratch

@@ -121,13 +121,13 @@ int merged_list_cap(const IntegShape& s);
 // wave.  Values as VDTTFS_PATH_* / vdttfs_layer_plan.
 // split (set by resolve_plan where the choice is the built-in one): forwards
 // without counters, with a LUT neuron and no fused pool take the split
-// integrator (1) or the column lists (2; k_split.hip) in place of the named
-// kernels.
+// integrator or the column lists (k_split.hip), or a pixel per lane
+// (k_pixel.hip, no scratch) in place of the named kernels.
 struct LaunchPlan {
     int path = 0, gather = 0, ppw = 0;
     int split = 0;
 };
-constexpr int kSplitDense = 1, kSplitLists = 2;
+constexpr int kSplitDense = 1, kSplitLists = 2, kSplitPixel = 3;
 constexpr int kMaxPixPerWave = 8;
 // The plan's lists come from the bin-layout bucketize (the bins and window paths).
 inline bool plan_bins(const LaunchPlan& p) { return p.path == VDTTFS_PATH_BINS || p.path == VDTTFS_PATH_WINDOW; }
@@ -186,6 +186,9 @@ int launch_integrate_dense(vdttfs_ctx* ctx, float* out, const float* in, const f
 // bins from per-column lists.  split_ok: the layers it can and should take;
 // split_scratch_bytes: the device scratch of one call.
 bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s);
+// The kernels of a layer without a plan of its own: a kSplit value, 0 for the
+// named plan's.
+int split_choice(const vdttfs_ctx* ctx, const IntegShape& s);
 size_t split_scratch_bytes(const IntegShape& s);
 int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
                            const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s);

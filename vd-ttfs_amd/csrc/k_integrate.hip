@@ -4137,9 +4137,7 @@ int resolve_named(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan&
 
 int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan& req, LaunchPlan* out) {
     VD_TRY(resolve_named(ctx, sh, req, out));
-    out->split = 0;
-    if (!req.path && !req.gather && !req.ppw)
-        out->split = split_ok(ctx, sh) ? kSplitDense : (lists_ok(ctx, sh) ? kSplitLists : 0);
+    out->split = !req.path && !req.gather && !req.ppw ? split_choice(ctx, sh) : 0;
     return VDTTFS_OK;
 }
 

@@ -1055,10 +1055,14 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
 // the register and narrow kernels do (batch 1024: conv1 145 against 567 us,
 // conv2 169 against 169).  Each group of four c_out blocks rebuilds a pixel's
 // list, so layers past 1024 outputs keep the merged lists.
-bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
-    // (fields past 32 elements that go without lists; smaller ones have a plan)
-    const bool px = conv_px_ok(s) && s.K_h * s.K_w * s.C_in > 32;
-    return (ctx->c.T > 64 || px) && lists_fit(ctx, s);
+bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64 && lists_fit(ctx, s); }
+
+int split_choice(const vdttfs_ctx* ctx, const IntegShape& s) {
+    // (up to 64 steps fields of at most 32 elements have a plan of their own)
+    if (conv_px_ok(s) && s.K_h * s.K_w <= kSplitMaxTaps && (ctx->c.T > 64 || s.K_h * s.K_w * s.C_in > 32))
+        return kSplitPixel;
+    if (split_ok(ctx, s)) return kSplitDense;
+    return lists_ok(ctx, s) ? kSplitLists : 0;
 }
 
 bool ref_lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return lists_fit(ctx, s); }
@@ -1208,8 +1212,6 @@ int launch_integrate_lists(vdttfs_ctx* ctx, float* out, const float* in, const f
                            const CulifNeuron* culif) {
     const int64_t cols = split_cols(s);
     if (cols == 0 || split_pix(s) == 0) return VDTTFS_OK;
-    // small fields go without lists (LeNet-5's conv1 at T = 80, batch 128: 78 -> 13 us)
-    if (!culif && conv_px_ok(s)) return launch_conv_px(ctx, out, in, alpha, W, bias, theta, t_min, s);
     LateScratch sc;
     carve(scratch, cols, s.C_in, &sc);
     VD_TRY(launch_split(ctx, SplitArgs{in, nullptr, sc.late, sc.cnt, alpha, theta, sc.thr, cols, s.C_in, s.C_in,

@@ -273,7 +273,9 @@ int forward_impl(vdttfs_net* net, const float* d_img, int32_t* d_pred, uint64_t*
             } else if (net->timing) {
                 VD_TRY(mark(net, &ti.a));
             }
-            if (split && plan.split == kSplitLists)
+            if (split && plan.split == kSplitPixel)
+                VD_TRY(launch_conv_px(ctx, l.out, cur, l.alpha, l.W, l.bias, l.theta, l.t_min, s));
+            else if (split && plan.split == kSplitLists)
                 VD_TRY(launch_integrate_lists(ctx, l.out, cur, l.alpha, net->list, l.W, l.bias, l.theta, l.t_min, s,
                                               nullptr));
             else if (split)
