@@ -111,8 +111,9 @@ int vdttfs_bucketize(vdttfs_ctx* ctx, const float* d_in, int64_t n_cols, int c_i
  * neuron never fires), NHWC with c_out fastest.  This is the reference-layout
  * export path, kept for bit-exact checks of caller-made buckets: the entries
  * are listed in context scratch and streamed a pixel per wave; past 25 taps,
- * 1024 outputs or 65535 weight rows, under stream capture, or without memory
- * for the lists one thread per neuron walks them.  vdttfs_layer_forward takes
+ * 1024 outputs or 65535 weight rows, without memory for the lists, or under
+ * stream capture where no earlier call has made the scratch large enough, one
+ * thread per neuron walks them.  vdttfs_layer_forward takes
  * the dense map.  Buckets are expected from this context's constants; events
  * outside their chunk's bins or the window, at cin >= C_in, and offsets past
  * the column are skipped / clamped rather than read out of range. */

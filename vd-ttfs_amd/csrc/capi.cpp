@@ -44,9 +44,23 @@ static int grow(void** p, size_t* have, size_t need_bytes) {
     return VDTTFS_OK;
 }
 
+// Waits for the stream's work on the scratch that is about to be replaced.
+// Under capture nothing may be waited for or allocated, and the capture stays
+// whole: the error says what to do.
+static int before_growth(vdttfs_ctx* ctx) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    VD_HIP(hipStreamIsCapturing(ctx->stream, &cs));
+    if (cs != hipStreamCaptureStatusNone)
+        return set_error(VDTTFS_E_UNSUPPORTED,
+                         "the context's scratch is too small and cannot grow under stream capture: run the call "
+                         "once before capturing it");
+    VD_HIP(hipStreamSynchronize(ctx->stream));
+    return VDTTFS_OK;
+}
+
 int ensure_ref_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols) {
     if (elems > ctx->ref_elems || cols > ctx->ref_cols || !ctx->ref_cin) {
-        VD_HIP(hipStreamSynchronize(ctx->stream));
+        VD_TRY(before_growth(ctx));
         size_t e = elems > ctx->ref_elems ? elems : ctx->ref_elems;
         size_t c = cols > ctx->ref_cols ? cols : ctx->ref_cols;
         size_t h1 = 0, h2 = 0, h3 = 0;
@@ -65,7 +79,7 @@ int ensure_ref_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols) {
 
 int ensure_bin_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols) {
     if (elems > ctx->bin_elems || cols > ctx->bin_cols || !ctx->bin_ev) {
-        VD_HIP(hipStreamSynchronize(ctx->stream));
+        VD_TRY(before_growth(ctx));
         size_t e = elems > ctx->bin_elems ? elems : ctx->bin_elems;
         size_t c = cols > ctx->bin_cols ? cols : ctx->bin_cols;
         size_t h1 = 0, h2 = 0;
@@ -97,7 +111,7 @@ int read_counters(vdttfs_ctx* ctx, unsigned long long out[4]) {
 
 int ensure_merge_scratch(vdttfs_ctx* ctx, size_t list_elems, size_t bstart_elems) {
     if (list_elems > ctx->mrg_list_elems || bstart_elems > ctx->mrg_bstart_elems || !ctx->mrg_list) {
-        VD_HIP(hipStreamSynchronize(ctx->stream));
+        VD_TRY(before_growth(ctx));
         size_t e = list_elems > ctx->mrg_list_elems ? list_elems : ctx->mrg_list_elems;
         size_t b = bstart_elems > ctx->mrg_bstart_elems ? bstart_elems : ctx->mrg_bstart_elems;
         size_t h1 = 0, h2 = 0;
@@ -113,15 +127,35 @@ int ensure_merge_scratch(vdttfs_ctx* ctx, size_t list_elems, size_t bstart_elems
     return VDTTFS_OK;
 }
 
-bool ensure_split_scratch(vdttfs_ctx* ctx, size_t list_elems) {
+bool ensure_split_scratch(vdttfs_ctx* ctx, size_t bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+    if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    if (ensure_merge_scratch(ctx, list_elems, 1) == VDTTFS_OK) return true;
-    (void)hipGetLastError();
-    return false;
+    const bool capturing = cs != hipStreamCaptureStatusNone;
+    if (ctx->split_buf && ctx->split_bytes >= bytes) {
+        ctx->split_captured |= capturing;
+        return true;
+    }
+    if (capturing || hipStreamSynchronize(ctx->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (ctx->split_captured)
+        ctx->split_kept.push_back(ctx->split_buf);
+    else if (ctx->split_buf)
+        (void)hipFree(ctx->split_buf);
+    ctx->split_buf = nullptr;
+    ctx->split_bytes = 0;
+    ctx->split_captured = false;
+    if (hipMalloc(&ctx->split_buf, bytes) != hipSuccess) {
+        ctx->split_buf = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    ctx->split_bytes = bytes;
+    return true;
 }
 
 static int check_consts(const vdttfs_consts* c) {
@@ -191,9 +225,10 @@ int vdttfs_destroy(vdttfs_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     void* bufs[] = {ctx->ref_cin, ctx->ref_tin,    ctx->ref_off,   ctx->bin_ev,
-                    ctx->bin_off, ctx->mrg_list, ctx->mrg_bstart, ctx->d_counters};
+                    ctx->bin_off, ctx->mrg_list, ctx->mrg_bstart, ctx->d_counters, ctx->split_buf};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
+    for (void* b : ctx->split_kept) (void)hipFree(b);
     if (ctx->timer_ready) {
         (void)hipEventDestroy(ctx->timer[0]);
         (void)hipEventDestroy(ctx->timer[1]);
@@ -367,19 +402,14 @@ static int engine_layer(vdttfs_ctx* ctx, float* d_out, const float* d_in, const 
     const int64_t cap = merged_list_cap(s);
     const bool dense = plan_from_dense(ctx, s, p, counters != nullptr);
     const bool lds_list = plan_lds_list(ctx, s, p, counters != nullptr, false);
-    if (p.split == kSplitPixel && !counters)  // no scratch
+    if (p.split == kSplitPixel && !counters)
         return launch_conv_px(ctx, d_out, d_in, d_lut_decay, d_kernel, d_bias, d_lut_th, t_min, s);
-    if (p.split && !counters) {
-        // as much as the named plan would take, so that a counting call of the
-        // layer finds its lists' scratch
-        const size_t need = split_scratch_bytes(s) / sizeof(int2) + 1, named = lds_list ? 0 : (size_t)(n_pix * cap);
-        if (ensure_split_scratch(ctx, need > named ? need : named))
-            return p.split == kSplitLists
-                       ? launch_integrate_lists(ctx, d_out, d_in, d_lut_decay, ctx->mrg_list, d_kernel, d_bias,
-                                                d_lut_th, t_min, s, nullptr)
-                       : launch_integrate_split(ctx, d_out, d_in, d_lut_decay, ctx->mrg_list, d_kernel, d_bias,
-                                                d_lut_th, t_min, s);
-    }
+    if (p.split && !counters && ensure_split_scratch(ctx, split_scratch_bytes(s)))
+        return p.split == kSplitLists
+                   ? launch_integrate_lists(ctx, d_out, d_in, d_lut_decay, ctx->split_buf, d_kernel, d_bias,
+                                            d_lut_th, t_min, s, nullptr)
+                   : launch_integrate_split(ctx, d_out, d_in, d_lut_decay, ctx->split_buf, d_kernel, d_bias,
+                                            d_lut_th, t_min, s);
     if (!lds_list)
         VD_TRY(ensure_merge_scratch(ctx, (size_t)(n_pix * cap), (size_t)n_pix * (ctx->c.T + 1)));
     if (dense)  // conv: merged lists straight from the dense map
@@ -409,8 +439,8 @@ int vdttfs_integrate(vdttfs_ctx* ctx, float* d_out, const int32_t* d_bkt_cin,
     // over every chunk's entries: 143 -> 13 us for 64->128, 3x3, 16x16, batch
     // 8 (several passes in flight), and ahead at every size tried, down to one
     // 5x5 map of 3 channels (37 -> 12 us a call)
-    if (ref_lists_ok(ctx, s) && ensure_split_scratch(ctx, split_scratch_bytes(s) / sizeof(int2) + 1))
-        return launch_integrate_ref_lists(ctx, d_out, d_bkt_cin, d_bkt_tin, d_bkt_off, ctx->mrg_list, d_kernel,
+    if (ref_lists_ok(ctx, s) && ensure_split_scratch(ctx, split_scratch_bytes(s)))
+        return launch_integrate_ref_lists(ctx, d_out, d_bkt_cin, d_bkt_tin, d_bkt_off, ctx->split_buf, d_kernel,
                                           d_bias, d_lut_decay, d_lut_th, t_min, s);
     return launch_integrate_ref(ctx, d_out, d_bkt_cin, d_bkt_tin, d_bkt_off, d_kernel, d_bias,
                                 d_lut_decay, d_lut_th, t_min, B, H_in, W_in, C_in, H_out, W_out,

@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <vector>
 
 #include "vdttfs.h"
 
@@ -35,6 +36,12 @@ struct vdttfs_ctx {
     void* mrg_list;
     void* mrg_bstart;
     size_t mrg_list_elems, mrg_bstart_elems;
+    // scratch of the split and list kernels.  split_captured: a captured graph
+    // holds its address, so growth sets it aside until the context ends
+    void* split_buf;
+    size_t split_bytes;
+    bool split_captured;
+    std::vector<void*> split_kept;
     unsigned long long* d_counters;  // kCounterStripes x 4 u64 (summed on the host)
     hipEvent_t timer[2];             // vdttfs_timer_begin/end (created on first use)
     bool timer_ready;
@@ -76,11 +83,11 @@ int check_ctx(vdttfs_ctx* ctx);
 int ensure_ref_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols);
 int ensure_bin_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols);
 int ensure_merge_scratch(vdttfs_ctx* ctx, size_t list_elems, size_t bstart_elems);
-// The split integrator's scratch, in the merged lists' buffer: at least
-// list_elems entries of it.  false where it cannot be had (no memory, or the
-// stream is under capture, whose replays must not depend on a buffer that a
-// later call may replace): the caller then takes the layer's other kernels.
-bool ensure_split_scratch(vdttfs_ctx* ctx, size_t list_elems);
+// The split and list kernels' scratch, ctx->split_buf: at least `bytes` of it.
+// false where it cannot be had (no memory, or the stream is under capture and
+// no earlier call has made it this large): the caller then takes the layer's
+// other kernels.
+bool ensure_split_scratch(vdttfs_ctx* ctx, size_t bytes);
 
 // ---- kernel launchers (stream-ordered on ctx->stream) ----
 int launch_encode_log(vdttfs_ctx* ctx, const float* img, float* out, int64_t n, float tc, float td);
