@@ -166,3 +166,26 @@ def test_capture_without_scratch_is_refused_whole(gpu_ctx_factory):
     ctx.synchronize()
     np.testing.assert_array_equal(out.download(), ref)
     g.close()
+
+
+def test_network_sizes_lists_for_the_layers_that_use_them(gpu_ctx_factory):
+    """An FC layer at T = 64 never takes the split kernels, whose scratch would
+    be half as large again as its merged lists (402 against 269 MB)."""
+    print("scratch network creation", flush=True)
+    B, cin, cout, T = 2048, 16384, 64, 64
+    ctx = gpu_ctx_factory(vdttfs.task2_consts(T=T, delta=8, tfs=32.0))
+    layer = vdttfs.Layer(vdttfs.LAYER_FC, 1, 1, cin, 1, 1, cout, kernel=np.zeros((cin, cout), np.float32),
+                         bias=np.zeros(cout, np.float32), tc_fire=16.0)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def free_bytes():
+        ctx.synchronize()
+        assert hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    before = free_bytes()
+    net = vdttfs.Net(ctx, [layer], B, cin, vdttfs.ENCODE_LINEAR, 16.0, 0.0, vdttfs.READOUT_ARGMIN)
+    used = before - free_bytes()
+    net.close()
+    lists, events, maps = B * (cin + 64) * 8, B * cin * 8, 4 * B * (cin + cout)
+    assert used < lists + events + maps + 4 * cin * cout + (64 << 20), used

@@ -267,6 +267,11 @@ int launch_fc_currents(vdttfs_ctx* ctx, const float* x, const float* W_t, float*
                        const FcSortScratch& sc);
 int launch_nhwc_to_nchw(vdttfs_ctx* ctx, const float* in, float* out, int N, int C, int H, int W);
 
+// A network's list buffer: `split` bytes for the split and list kernels where
+// they need more than the named plans' `named` bytes, and those alone where
+// that much cannot be had (the layers that need more then take their plans).
+int list_alloc(void** p, size_t named, size_t split, size_t* bytes);
+
 // Layer-table checks of vdttfs_net_create (shapes chain, kinds, weights).
 int validate_layer_table(const vdttfs_consts& c, const vdttfs_layer_desc* layers, int n, int64_t img_elems);
 

@@ -59,6 +59,7 @@ struct vdttfs_culif_net {
     vd_event* ev = nullptr;    // bin-layout events
     int32_t* off = nullptr;    // bin offsets
     int2* list = nullptr;      // merged lists
+    size_t list_bytes = 0;
     int32_t* bstart = nullptr;
     int32_t* rcin = nullptr;   // reference-layout buckets (small FC)
     float* rtin = nullptr;
@@ -153,6 +154,7 @@ int create_impl(vdttfs_culif_net* net, const vdttfs_culif_layer* layers, int n) 
     std::vector<float> ones(T + 1, 1.0f);
     VD_TRY(upload(&net->ones, ones));
     int64_t max_ev = 1, max_cols = 1, max_list = 1, max_bstart = 1, max_flat = 1, max_cur = 1;
+    size_t split_bytes = 0;
     int64_t max_fc_counts = 1, max_fc_binstart = 1, max_fc_list = 1;
     int64_t max_rsites = 1, max_relems = 1;
     net->L.resize(n);
@@ -203,8 +205,7 @@ int create_impl(vdttfs_culif_net* net, const vdttfs_culif_layer* layers, int n) 
                 if (cols * d.C_in > max_ev) max_ev = cols * d.C_in;
                 if (cols > max_cols) max_cols = cols;
                 if (n_pix * l.list_cap > max_list) max_list = n_pix * l.list_cap;
-                const int64_t split_list = (int64_t)(split_scratch_bytes(sh) / sizeof(int2)) + 1;
-                if (split_list > max_list) max_list = split_list;
+                if (lists_ok(ctx, sh) && split_scratch_bytes(sh) > split_bytes) split_bytes = split_scratch_bytes(sh);
                 if (n_pix * (T + 1) > max_bstart) max_bstart = n_pix * (T + 1);
                 break;
             }
@@ -246,7 +247,6 @@ int create_impl(vdttfs_culif_net* net, const vdttfs_culif_layer* layers, int n) 
     const int OS = T / ctx->c.delta + 1;
     VD_TRY(dalloc((void**)&net->ev, (size_t)max_ev * sizeof(vd_event)));
     VD_TRY(dalloc((void**)&net->off, (size_t)max_cols * (T + 1) * 4));
-    VD_TRY(dalloc((void**)&net->list, (size_t)max_list * sizeof(int2)));
     VD_TRY(dalloc((void**)&net->bstart, (size_t)max_bstart * 4));
     VD_TRY(dalloc((void**)&net->rcin, (size_t)max_relems * 4));
     VD_TRY(dalloc((void**)&net->rtin, (size_t)max_relems * 4));
@@ -257,6 +257,7 @@ int create_impl(vdttfs_culif_net* net, const vdttfs_culif_layer* layers, int n) 
     VD_TRY(dalloc((void**)&net->fcs.offs, (size_t)max_fc_counts * 4));
     VD_TRY(dalloc((void**)&net->fcs.binstart, (size_t)max_fc_binstart * 4));
     VD_TRY(dalloc((void**)&net->fcs.list, (size_t)max_fc_list * 4));
+    VD_TRY(list_alloc((void**)&net->list, (size_t)max_list * sizeof(int2), split_bytes, &net->list_bytes));
     return VDTTFS_OK;
 }
 
@@ -316,7 +317,7 @@ int forward_impl(vdttfs_culif_net* net, const float* d_data, int32_t* d_pred, ui
                 // map (the bin-layout bucketize then only counts retained events)
                 LaunchPlan plan;
                 VD_TRY(resolve_plan(ctx, sh, LaunchPlan{}, &plan));
-                if (!count_here && ctx->c.T > 64 && lists_ok(ctx, sh)) {
+                if (!count_here && lists_ok(ctx, sh) && split_scratch_bytes(sh) <= net->list_bytes) {
                     VD_TRY(launch_integrate_lists(ctx, l.out, cur, net->ones, net->list, l.W, nullptr, nullptr, 0, sh,
                                                   &nrn));
                     break;

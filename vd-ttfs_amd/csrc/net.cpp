@@ -69,6 +69,7 @@ struct vdttfs_net {
     vd_event* ev = nullptr;
     int32_t* off = nullptr;
     int2* list = nullptr;
+    size_t list_bytes = 0;
     int32_t* bstart = nullptr;
     bool timing = false;
     int pool_fusion = VDTTFS_POOL_FUSE_OFF;  // which 2x2 pools run inside the next layer's list build
@@ -255,8 +256,10 @@ int forward_impl(vdttfs_net* net, const float* d_img, int32_t* d_pred, uint64_t*
             LaunchPlan plan;
             VD_TRY(resolve_plan(ctx, s, l.plan, &plan));
             // the built-in choice of layers with a late fire start or a long
-            // window; its scratch is the merged lists' (sized for both at creation)
-            const bool split = plan.split && !count && !fuse;
+            // window; its scratch is the merged lists' (sized for both at
+            // creation, where there was the memory)
+            const bool split = plan.split && !count && !fuse &&
+                               (plan.split == kSplitPixel || split_scratch_bytes(s) <= net->list_bytes);
             const bool dense = split || plan_from_dense(ctx, s, plan, count);
             TimedPair tb{}, ti{};
             tb.layer = ti.layer = (int)i;
@@ -357,11 +360,23 @@ int dalloc(void** p, size_t bytes) {
     return VDTTFS_OK;
 }
 
+// The split and list kernels' scratch of a layer: 0 where no window up to the
+// context's (set_windows) lets it take them.
+size_t net_split_bytes(vdttfs_ctx* ctx, const IntegShape& s) {
+    for (int t = ctx->c.T; t >= 1; --t) {
+        WindowScope window(ctx, t);
+        const int k = split_choice(ctx, s);
+        if (k == kSplitDense || k == kSplitLists) return split_scratch_bytes(s);
+    }
+    return 0;
+}
+
 int create_impl(vdttfs_net* net, const vdttfs_layer_desc* layers, int n) {
     vdttfs_ctx* ctx = net->ctx;
     const vdttfs_consts& c = ctx->c;
     VD_TRY(dalloc((void**)&net->enc, (size_t)net->B * net->img_elems * 4));
     int64_t max_elems = 1, max_cols = 1, max_list = 1, max_bstart = 1;
+    size_t split_bytes = 0;
     float tc_i = net->tc_in, td_i = net->td_in;
     std::vector<float> ha(c.T + 1), ht(c.T);
     net->L.resize(n);
@@ -409,15 +424,15 @@ int create_impl(vdttfs_net* net, const vdttfs_layer_desc* layers, int n) {
         l.list_cap = merged_list_cap(s);
         const int64_t n_pix = (int64_t)net->B * (fc ? 1 : (int64_t)d.H_out * d.W_out);
         if (n_pix * l.list_cap > max_list) max_list = n_pix * l.list_cap;
-        const int64_t split_list = (int64_t)(split_scratch_bytes(s) / sizeof(int2)) + 1;
-        if ((c.tfs > 0.0f || c.T > 64) && split_list > max_list) max_list = split_list;
+        const size_t sb = net_split_bytes(ctx, s);
+        if (sb > split_bytes) split_bytes = sb;
         if (n_pix * (c.T + 1) > max_bstart) max_bstart = n_pix * (c.T + 1);
     }
     for (int i = 0; i < n; ++i) net->L[i].d.kernel = net->L[i].d.bias = nullptr;
     VD_TRY(dalloc((void**)&net->ev, (size_t)max_elems * sizeof(vd_event)));
     VD_TRY(dalloc((void**)&net->off, (size_t)max_cols * (c.T + 1) * 4));
-    VD_TRY(dalloc((void**)&net->list, (size_t)max_list * sizeof(int2)));
     VD_TRY(dalloc((void**)&net->bstart, (size_t)max_bstart * 4));
+    VD_TRY(list_alloc((void**)&net->list, (size_t)max_list * sizeof(int2), split_bytes, &net->list_bytes));
     VD_HIP(hipDeviceSynchronize());
     return VDTTFS_OK;
 }
@@ -425,6 +440,17 @@ int create_impl(vdttfs_net* net, const vdttfs_layer_desc* layers, int n) {
 }  // namespace
 
 namespace vdttfs {
+int list_alloc(void** p, size_t named, size_t split, size_t* bytes) {
+    if (split > named && hipMalloc(p, split) == hipSuccess) {
+        *bytes = split;
+        return VDTTFS_OK;
+    }
+    (void)hipGetLastError();
+    VD_TRY(dalloc(p, named));
+    *bytes = named;
+    return VDTTFS_OK;
+}
+
 int validate_layer_table(const vdttfs_consts& c, const vdttfs_layer_desc* layers, int n, int64_t img_elems) {
     return validate(c, layers, n, img_elems);
 }
