@@ -30,6 +30,12 @@ SHAPES = [
     ("t64-conv3-12-13-same", 64, 9, True, False, 9, 31, 30, 12, 13, 3),
     ("t64-conv5-6-16", 64, 0, False, False, 90, 31, 32, 6, 16, 5),
     ("t140-conv1-160-10", 140, 0, True, False, 80, 29, 29, 160, 10, 1),
+    # nine outputs and more up to 64 steps: a lane per output below 12,288 pixels
+    ("t64-conv5-1-16-few", 64, 0, False, False, 15, 32, 32, 1, 16, 5),
+    ("t64-conv5-1-16-many", 64, 0, False, False, 16, 32, 32, 1, 16, 5),
+    ("t64-conv3-3-9-same-few", 64, 0, True, False, 12, 32, 31, 3, 9, 3),
+    ("t64-conv3-3-9-same-many", 64, 0, True, False, 13, 32, 31, 3, 9, 3),
+    ("t64-conv1-16-10-few", 64, 0, True, False, 2, 9, 7, 16, 10, 1),
 ]
 KINDS = ["random", "silent", "bin0", "last-bin", "dense", "fractional"]
 

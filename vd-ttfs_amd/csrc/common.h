@@ -204,7 +204,7 @@ int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const f
 // 64 steps); in split_scratch_bytes of scratch.
 bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s);
 // Small fields and few outputs, one pixel per lane (k_pixel.hip).
-bool conv_px_ok(const IntegShape& s);
+bool conv_px_ok(int T, const IntegShape& s);
 int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W, const float* bias,
                    const float* theta, int t_min, const IntegShape& s);
 // ... and over the reference's buckets.

@@ -3845,9 +3845,10 @@ bool small_ok(const vdttfs_ctx* ctx, const IntegShape& sh) {
 
 int launch_conv_small(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W,
                       const float* bias, const float* theta, int t_min, const IntegShape& sh) {
-    // up to 16 outputs a lane holds all of a pixel (LeNet-5's conv1, batch
-    // 1024: 145 -> 34 us); wider layers would leave too few registers
-    if (conv_px_ok(sh)) return launch_conv_px(ctx, out, in, alpha, W, bias, theta, t_min, sh);
+    // up to 16 outputs, where the pixels are enough, a lane holds all of a pixel
+    // (LeNet-5's conv1, batch 1024: 145 -> 34 us); wider layers would leave too
+    // few registers
+    if (conv_px_ok(ctx->c.T, sh)) return launch_conv_px(ctx, out, in, alpha, W, bias, theta, t_min, sh);
     SmallArgs a{};
     a.in = in;
     a.alpha = alpha;

@@ -240,22 +240,34 @@ __global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
 
 }  // namespace
 
+// Up to 32 elements, past 64 steps: against lists in memory, at every size
+// (LeNet-5's conv1 at T = 80, batch 128: 78 -> 13 us).  Up to 64 steps
+// k_conv_small spreads a pixel's outputs over lanes and finishes first where
+// outputs are many and pixels leave the chip idle (us a call, k_conv_small
+// against this; a fifth of the inputs active):
+//   25 elements, 16 outputs:  4,096 pixels 12.9 / 15.3, 12,544 17.8 / 16.2
+//   27 elements, 16 outputs:  4,096 pixels 15.8 / 17.5, 12,544 23.4 / 18.2
+//   25 elements, 8 outputs:   784 pixels 12.5 / 11.3;  16 and 16: 12.5 / 12.8
 // Past 32 elements the search costs more than a list, which finds its order
-// once, unless the pixels fill the chip: k_merge_dense + k_stream_narrow
-// against this, T = 64: 108 elements, 16K pixels 50 -> 39 us (density 0.5) and
-// 40 -> 23 (0.1); 150 elements, 66K pixels 168 -> 136, but 33K pixels 95 ->
-// 120.
-bool conv_px_ok(const IntegShape& s) {
+// once, unless the pixels are many: k_merge_dense + k_stream_narrow against
+// this, T = 64: 108 elements, 16K pixels 50 -> 39 us (density 0.5) and 40 ->
+// 23 (0.1), at 8K 0.8 to 1.3 times the speed; 150 elements, LeNet-5's conv2:
+// 66K pixels 168 -> 136.  The line for those lies where a workgroup has four
+// waves (launch_conv_px): with one, each wave loads the weights for itself, and
+// LeNet-5 takes 7 to 13% longer a pass at 45K to 64K pixels (batches 700 to
+// 1000, T = 64; with three passes in flight they are even).
+bool conv_px_ok(int T, const IntegShape& s) {
     const int64_t in = (int64_t)s.B * s.H_in * s.W_in * s.C_in * 4, pix = (int64_t)s.B * s.H_out * s.W_out;
     const int64_t nel = (int64_t)s.K_h * s.K_w * s.C_in;
     if (s.is_fc || s.C_out > kPxMaxOut || nel > kPxMaxEl) return false;
     if (in >= (INT64_C(1) << 31) || 4 * pix >= (INT64_C(1) << 31) - 256) return false;
-    return nel <= 32 || pix >= (nel <= 112 ? 8192 : 65536);
+    if (nel > 32) return pix >= (nel <= 112 ? 8192 : 65536);
+    return T > 64 || s.C_out <= 8 || nel <= 16 || pix >= 12288;
 }
 
 int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W, const float* bias,
                    const float* theta, int t_min, const IntegShape& s) {
-    if (!conv_px_ok(s) || ctx->c.T > 255) return set_error(VDTTFS_E_UNSUPPORTED, "conv_px: layer outside its limits");
+    if (!conv_px_ok(ctx->c.T, s) || ctx->c.T > 255) return set_error(VDTTFS_E_UNSUPPORTED, "conv_px: layer outside its limits");
     PxArgs a{};
     a.in = in;
     a.alpha = alpha;

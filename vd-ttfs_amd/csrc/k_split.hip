@@ -1059,7 +1059,7 @@ bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64
 
 int split_choice(const vdttfs_ctx* ctx, const IntegShape& s) {
     // (up to 64 steps fields of at most 32 elements have a plan of their own)
-    if (conv_px_ok(s) && s.K_h * s.K_w <= kSplitMaxTaps && (ctx->c.T > 64 || s.K_h * s.K_w * s.C_in > 32))
+    if (conv_px_ok(ctx->c.T, s) && s.K_h * s.K_w <= kSplitMaxTaps && (ctx->c.T > 64 || s.K_h * s.K_w * s.C_in > 32))
         return kSplitPixel;
     if (split_ok(ctx, s)) return kSplitDense;
     return lists_ok(ctx, s) ? kSplitLists : 0;
