@@ -1,12 +1,15 @@
 """The split integrator (bin 0 on the matrix cores, the later bins from
 per-column lists) against the oracle, bit for bit.
 
-The layers are of the sizes the built-in choice gives it: past 64 steps (any
-size), past 9 taps, long fields.  They cross partial pixel and c_out tiles of
-every tile size, odd C_out (one load per column), C_in outside multiples of 8
-and 16, every tap count's kernel, two bin blocks, lists past a window's
-capacity, thresholds that are not monotone, non-finite weights, t_min > 0,
-valid and same padding, and FC layers.
+SHAPES are layers of all kinds with few pixels: one to 25 taps, two bin blocks,
+odd C_out (one load per column), C_in outside multiples of 8 and 16, lists past
+a window's capacity, thresholds that are not monotone, non-finite weights,
+t_min > 0, valid and same padding, and FC layers.  Those that the split takes
+run its 16x16 tiles; the others run on the fused kernels or the column lists
+and are compared all the same.  TILES are layers that the split takes (checked
+against its size rule), with each tile of its matrix product: odd and even
+C_out past whole tiles, C_in outside multiples of 8, partial pixel tiles, rows
+in image and in (position, image) order, non-finite weights.
 """
 import sys
 import zlib
@@ -33,7 +36,22 @@ SHAPES = [
     ("t48-conv3-256-256", 48, 24, True, False, 3, 3, 2, 256, 256, 3),
     ("t80-fc-600-260", 80, 40, True, True, 19, 1, 1, 600, 260, 1),
     ("t65-fc-30-40", 65, 17, False, True, 70, 1, 1, 30, 40, 1),
-    ("t64-conv3-64-64-big", 64, 32, True, False, 40, 16, 16, 64, 64, 3),   # 64x64 tiles
+    ("t64-conv3-64-64-big", 64, 32, True, False, 40, 16, 16, 64, 64, 3),
+]
+# k_gemm0's tile of a wave (pixels x c_out), then a shape that takes it
+TILES = [
+    ((16, 16), ("t64-conv5-5-33-small", 64, 32, True, False, 7, 6, 7, 5, 33, 5)),
+    ((16, 16), ("t128-conv3-36-131", 128, 64, True, False, 2, 6, 7, 36, 131, 3)),         # two bin blocks
+    ((32, 32), ("t64-conv5-5-33", 64, 32, True, False, 147, 13, 11, 5, 33, 5)),
+    ((32, 32), ("t64-conv5-3-34", 64, 32, False, False, 149, 13, 14, 3, 34, 5)),
+    ((32, 32), ("t64-conv5-5-33-pos", 64, 32, True, False, 353, 5, 7, 5, 33, 5)),         # (position, image) rows
+    ((32, 32), ("t64-conv3-20-70", 64, 32, True, False, 58, 13, 11, 20, 70, 3)),          # nine taps
+    ((32, 64), ("t64-conv5-5-67", 64, 32, True, False, 153, 13, 11, 5, 67, 5)),
+    ((32, 64), ("t64-conv5-3-66", 64, 16, True, False, 153, 13, 11, 3, 66, 5)),
+    ((32, 64), ("t64-conv5-5-67-pos", 64, 32, True, False, 645, 5, 7, 5, 67, 5)),
+    ((64, 64), ("t64-conv5-2-131", 64, 32, True, False, 737, 13, 11, 2, 131, 5)),
+    ((64, 64), ("t64-conv5-2-130", 64, 32, True, False, 737, 13, 11, 2, 130, 5)),
+    ((64, 64), ("t64-conv5-2-131-pos", 64, 32, True, False, 3001, 5, 7, 2, 131, 5)),
 ]
 KINDS = ["random", "silent", "bin0", "one-late-bin", "last-bin", "late", "dense", "fractional"]
 
@@ -98,6 +116,55 @@ def test_split_matches_oracle(gpu_ctx_factory, shape, kind):
         assert (ref < INF).any() and (ref == INF).any(), "the case must fire some neurons and not others"
     got = run(gpu_ctx_factory(tc), shape, ho, wo, Wt, bias, sp, alpha, theta, 3)
     np.testing.assert_array_equal(got, ref, err_msg=f"{shape[0]} {kind}")
+
+
+def tile_of(shape):
+    """The split's tile for a layer, or None where the split does not take it
+    (its rules on sizes for at most 25 taps)."""
+    _, T, tfs, task2, is_fc, B, H, W, C_in, C_out, K = shape
+    taps = 1 if is_fc else K * K
+    pix = B * (1 if is_fc else (H * W if task2 else (H - K + 1) * (W - K + 1)))
+    nel = taps * C_in
+    tiles = -(-pix // 32) * -(-C_out // 32)
+    if C_out < 32 or 4 * tfs < T or T > 128:
+        return None
+    if T > 64 or taps > 9:
+        if nel < 4:
+            return None
+    elif is_fc or tiles < 768 or nel < 144 or nel * pix * C_out < 10**8 or (2 * tfs < T and tiles < 4096):
+        return None
+    return (64, 64) if tiles >= 16384 else (32, 64) if tiles >= 2048 else (32, 32) if tiles >= 768 else (16, 16)
+
+
+@pytest.mark.parametrize("kind", ["random", "bin0", "fractional"])
+@pytest.mark.parametrize("tile,shape", TILES, ids=[t[1][0] for t in TILES])
+def test_split_tiles(gpu_ctx_factory, tile, shape, kind):
+    assert tile_of(shape) == tile
+    test_split_matches_oracle(gpu_ctx_factory, shape, kind)
+
+
+LINES = [  # either side of the lines that the split is chosen by up to 64 steps and nine taps
+    ((32, 32), ("t64-conv3-20-70-768", 64, 32, True, False, 16, 32, 16, 20, 70, 3)),
+    (None, ("t64-conv3-20-70-767", 64, 32, True, False, 15, 34, 16, 20, 70, 3)),
+    (None, ("t64-conv3-20-70-early", 64, 31, True, False, 16, 32, 16, 20, 70, 3)),
+    ((32, 64), ("t64-conv3-20-66-early", 64, 31, True, False, 45, 31, 32, 20, 66, 3)),
+    (None, ("t64-conv3-15-99", 64, 32, True, False, 16, 32, 16, 15, 99, 3)),
+    ((32, 32), ("t64-conv3-16-99", 64, 32, True, False, 16, 32, 16, 16, 99, 3)),
+]
+
+
+@pytest.mark.parametrize("tile,shape", LINES, ids=[t[1][0] for t in LINES])
+def test_split_lines(gpu_ctx_factory, tile, shape):
+    assert tile_of(shape) == tile
+    test_split_matches_oracle(gpu_ctx_factory, shape, "random")
+
+
+@pytest.mark.parametrize("what", ["inf-weight", "nan-weight", "inf-row0"])
+@pytest.mark.parametrize("tile,shape", [TILES[k] for k in (2, 4, 7, 8, 9, 10)],
+                         ids=[TILES[k][1][0] for k in (2, 4, 7, 8, 9, 10)])
+def test_split_tiles_non_finite_weights(gpu_ctx_factory, tile, shape, what):
+    assert tile_of(shape) == tile
+    test_split_odd_tables_and_weights(gpu_ctx_factory, shape, what)
 
 
 @pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[4], SHAPES[7]], ids=lambda s: s[0])

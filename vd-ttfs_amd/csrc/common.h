@@ -145,7 +145,7 @@ bool plan_lds_list(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan
 // Fills every field of *out: a requested field is checked against the
 // layer's shape (VDTTFS_E_UNSUPPORTED when the kernels cannot run it), a zero
 // field takes the built-in choice.
-int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& s, const LaunchPlan& req, LaunchPlan* out);
+int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& s, const LaunchPlan& req, LaunchPlan* out, bool net = false);
 
 // Engine integrator over the bin layout: merge per pixel, then stream.
 // list/bstart: merged-list scratch of n_pix*list_cap entries and
@@ -192,10 +192,11 @@ int launch_integrate_dense(vdttfs_ctx* ctx, float* out, const float* in, const f
 // The split integrator (k_split.hip): bin 0 on the matrix cores, the later
 // bins from per-column lists.  split_ok: the layers it can and should take;
 // split_scratch_bytes: the device scratch of one call.
-bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s);
+bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s, bool net);
 // The kernels of a layer without a plan of its own: a kSplit value, 0 for the
-// named plan's.
-int split_choice(const vdttfs_ctx* ctx, const IntegShape& s);
+// named plan's.  net: a network's layer, whose inputs are spikes of the layer
+// before, rather than a call with a map of any kind.
+int split_choice(const vdttfs_ctx* ctx, const IntegShape& s, bool net);
 size_t split_scratch_bytes(const IntegShape& s);
 int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, void* scratch,
                            const float* W, const float* bias, const float* theta, int t_min, const IntegShape& s);

@@ -4136,9 +4136,9 @@ int resolve_named(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan&
 
 }  // namespace
 
-int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan& req, LaunchPlan* out) {
+int resolve_plan(const vdttfs_ctx* ctx, const IntegShape& sh, const LaunchPlan& req, LaunchPlan* out, bool net) {
     VD_TRY(resolve_named(ctx, sh, req, out));
-    out->split = !req.path && !req.gather && !req.ppw ? split_choice(ctx, sh) : 0;
+    out->split = !req.path && !req.gather && !req.ppw ? split_choice(ctx, sh, net) : 0;
     return VDTTFS_OK;
 }
 

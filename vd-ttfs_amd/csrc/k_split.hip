@@ -974,9 +974,11 @@ int ceil16(int c) { return (c + 15) & ~15; }
 int64_t split_cols(const IntegShape& s) { return s.is_fc ? s.B : (int64_t)s.B * s.H_in * s.W_in; }
 int64_t split_pix(const IntegShape& s) { return s.is_fc ? s.B : (int64_t)s.B * s.H_out * s.W_out; }
 
-// k_gemm0's tiles: 0: 64 x 64 a wave (2 x 2 of 32x32), 1: 32 x 64, 2: 32 x 32, 3: 16 x 16.
+// k_gemm0's tiles: 0: 64 x 64 a wave (2 x 2 of 32x32), 1: 32 x 64, 2: 32 x 32, 3: 16 x 16, by the 32x32 tiles of
+// the layer.
+int64_t tiles32(int64_t pix, int c_out) { return ((pix + 31) / 32) * ((c_out + 31) / 32); }
 int gemm0_config(int64_t pix, int c_out) {
-    const int64_t tiles = ((pix + 31) / 32) * ((c_out + 31) / 32);  // of 32 x 32
+    const int64_t tiles = tiles32(pix, c_out);
     return tiles >= 16384 ? 0 : (tiles >= 2048 ? 1 : (tiles >= 768 ? 2 : 3));
 }
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
@@ -995,7 +997,7 @@ size_t split_scratch_bytes(const IntegShape& s) {
            align256(sizeof(LateThr));
 }
 
-bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
+bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
     const int T = ctx->c.T;
     const int taps = s.is_fc ? 1 : s.K_h * s.K_w;
     const int64_t cols = split_cols(s), pix = split_pix(s), K = (int64_t)taps * s.C_in;
@@ -1006,9 +1008,7 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
     if (!late_grid_ok(pix, s.C_out)) return false;
     // Bin 0 collects the spikes up to the fire start: from a quarter of the
     // window on it holds enough of them that the dense sum beats the gather
-    // (VGG-16's layers hold 70-85% there at half the window; layers with a
-    // tenth of their inputs active, 5% in bin 0, still gain 1.4-2.5x past the
-    // sizes below).
+    // (VGG-16's layers hold 70-85% there at half the window).
     if (!(ctx->c.tfs * 4.0f >= (float)T)) return false;
     // Three launches and the element chain of k_gemm0 (32 cycles an element,
     // 8 in 16x16 tiles) need work to hide under.  Where the fused kernels do
@@ -1021,11 +1021,37 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
     // pixels, whose taps mostly fall outside (512 -> 512 at B=128: 54 against
     // 57 us; B=256: 98 -> 91).
     if (s.is_fc || (s.H_out * s.W_out <= 4 && pix < 1024)) return false;
-    // Past 10^8 products (conv 64 -> 64 at 4,096 pixels 30 -> 27 us, at 1,024
-    // pixels 21 against 24; 63 inputs x 79 outputs at 2,760 pixels 14.6
-    // against 18.6), or with long fields, which the fused kernels stream one
-    // event after the other (VGG-16 at B=1: 128 -> 256 on 8x8 38 -> 29 us).
-    return K * pix * s.C_out >= 100000000 || (K >= 1024 && s.C_out > 64);
+    // The dense sum costs the same at any density, so the line depends on what
+    // arrives, which the host does not see.
+    const int64_t products = K * pix * s.C_out;
+    if (net) {
+        // Layers of a network: most of their inputs spike before the fire
+        // start.  Past 10^8 products, or with long fields, which the fused
+        // kernels stream one event after the other (VGG-16 at B=1: 128 -> 256
+        // on 8x8 38 -> 29 us, 512 -> 512 on 4x4 1.2 to 1.4 times as fast).
+        // Weights past an XCD's L2 (4 MB) come from the Infinity Cache once per
+        // row of 16-pixel tiles, which costs more than the events where
+        // neither pixels nor chains hide it (VGG-16 with its 4x4 layers split
+        // against fused, us a pass alone and of three in flight: B=3 544 / 575,
+        // 237 / 232; B=4 570 / 576, 258 / 237; B=8 585 / 584, 288 / 261; B=16
+        // 645 / 645, 359 / 354; B=24 744 / 772, 469 / 485).
+        if (K * s.C_out > (1 << 20) && pix > 48 && pix < 384) return false;
+        return products >= 100000000 || (K >= 1024 && s.C_out > 64);
+    }
+    // Single layers, spikes spread over the window (half of them in bin 0):
+    // from 768 tiles of 32x32 on, where k_gemm0 takes those (split against
+    // fused, times as fast at densities 0.1 / 0.3 / 0.7, alone: 64 -> 64 at 16K
+    // pixels 1.0 / 1.16 / 1.22, 128 -> 256 at 4K 0.83 / 1.06 / 1.27, 72 -> 100
+    // at 8K 0.92 / 1.08 / 1.17, 64 -> 128 at 64K 1.07 / 1.25 / 1.32).  Below, with
+    // 16x16 tiles, it loses at most densities (128 -> 128 at 4K 0.65 / 0.83 /
+    // 1.02, at 1K 0.77 / 0.88 / 0.92; 190 -> 239 at 1K 0.72 / 0.94 / 1.14), more
+    // with several passes in flight, and so do short chains (1x1, 128 -> 128 at
+    // 8K 0.71 / 0.79 / 0.90) and, on fewer than 4,096 tiles, fire starts in the
+    // window's first half (a quarter: 128 -> 256 at 8K 0.86 / 0.94 / 1.05).
+    const int64_t tiles = tiles32(pix, s.C_out);
+    if (tiles < 768 || products < 100000000) return false;
+    if (K < 144 && products < 1000000000) return false;
+    return ctx->c.tfs * 2.0f >= (float)T || tiles >= 4096;
 }
 
 namespace {
@@ -1057,11 +1083,11 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
 // list, so layers past 1024 outputs keep the merged lists.
 bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64 && lists_fit(ctx, s); }
 
-int split_choice(const vdttfs_ctx* ctx, const IntegShape& s) {
+int split_choice(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
     // (up to 64 steps fields of at most 32 elements have a plan of their own)
     if (conv_px_ok(ctx->c.T, s) && s.K_h * s.K_w <= kSplitMaxTaps && (ctx->c.T > 64 || s.K_h * s.K_w * s.C_in > 32))
         return kSplitPixel;
-    if (split_ok(ctx, s)) return kSplitDense;
+    if (split_ok(ctx, s, net)) return kSplitDense;
     return lists_ok(ctx, s) ? kSplitLists : 0;
 }
 

@@ -254,7 +254,7 @@ int forward_impl(vdttfs_net* net, const float* d_img, int32_t* d_pred, uint64_t*
             // the dense map; the bin-layout bucketize runs for the bins path,
             // and in a counting forward for its retained-event count
             LaunchPlan plan;
-            VD_TRY(resolve_plan(ctx, s, l.plan, &plan));
+            VD_TRY(resolve_plan(ctx, s, l.plan, &plan, /*net=*/true));
             // the built-in choice of layers with a late fire start or a long
             // window; its scratch is the merged lists' (sized for both at
             // creation, where there was the memory)
@@ -365,7 +365,7 @@ int dalloc(void** p, size_t bytes) {
 size_t net_split_bytes(vdttfs_ctx* ctx, const IntegShape& s) {
     for (int t = ctx->c.T; t >= 1; --t) {
         WindowScope window(ctx, t);
-        const int k = split_choice(ctx, s);
+        const int k = split_choice(ctx, s, /*net=*/true);
         if (k == kSplitDense || k == kSplitLists) return split_scratch_bytes(s);
     }
     return 0;
