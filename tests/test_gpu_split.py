@@ -128,7 +128,10 @@ def tile_of(shape):
     tiles = -(-pix // 32) * -(-C_out // 32)
     if C_out < 32 or 4 * tfs < T or T > 128:
         return None
-    if T > 64 or taps > 9:
+    if T > 64:
+        if nel <= 300:
+            return None
+    elif taps > 9:
         if nel < 4:
             return None
     elif is_fc or tiles < 768 or nel < 144 or nel * pix * C_out < 10**8 or (2 * tfs < T and tiles < 4096):
@@ -143,11 +146,13 @@ def test_split_tiles(gpu_ctx_factory, tile, shape, kind):
     test_split_matches_oracle(gpu_ctx_factory, shape, kind)
 
 
-LINES = [  # either side of the lines that the split is chosen by up to 64 steps and nine taps
+LINES = [  # either side of the lines that the split is chosen by
     ((32, 32), ("t64-conv3-20-70-768", 64, 32, True, False, 16, 32, 16, 20, 70, 3)),
     (None, ("t64-conv3-20-70-767", 64, 32, True, False, 15, 34, 16, 20, 70, 3)),
     (None, ("t64-conv3-20-70-early", 64, 31, True, False, 16, 32, 16, 20, 70, 3)),
     ((32, 64), ("t64-conv3-20-66-early", 64, 31, True, False, 45, 31, 32, 20, 66, 3)),
+    (None, ("t80-conv5-12-40", 80, 40, True, False, 2, 9, 7, 12, 40, 5)),  # 300 elements: column lists
+    ((16, 16), ("t80-conv1-301-40", 80, 40, True, False, 3, 9, 7, 301, 40, 1)),
     (None, ("t64-conv3-15-99", 64, 32, True, False, 16, 32, 16, 15, 99, 3)),
     ((32, 32), ("t64-conv3-16-99", 64, 32, True, False, 16, 32, 16, 16, 99, 3)),
 ]

@@ -1013,9 +1013,15 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
     // Three launches and the element chain of k_gemm0 (32 cycles an element,
     // 8 in 16x16 tiles) need work to hide under.  Where the fused kernels do
     // not serve (T > 64, or more than 9 taps: bucketize or dense merge and a
-    // stream) that is any layer of a few inputs: 48 inputs x 116 outputs at
-    // 3,069 pixels 26.6 -> 17.4 us.
-    if (T > 64 || taps > 9) return K >= 4;
+    // stream) that is any layer of a few inputs past nine taps.
+    if (T <= 64 && taps > 9) return K >= 4;
+    // Past 64 steps the lists of every bin (two launches) are there as well and
+    // finish first in short fields, where the split even lost to the kernels
+    // before it (3x3, C_in 3, 64 outputs, T = 80, 1,024 pixels, us at densities
+    // 0.1 / 0.7: dense merge and stream 11.9 / 16.0, split 14.9 / 15.4, lists
+    // 8.4 / 9.2; times as fast as the split: 72 elements 1.75 / 1.6, 171 1.7 /
+    // 1.35, 300 1.9 / 1.2, 576 1.7 / 1.06 there and 1.5 / 0.8 at 16K pixels).
+    if (T > 64) return K > 300;
     // Against the fused kernels: FC layers keep them (VGG-16's 512 -> 512 at
     // B=256: 28 against 34 us), and so do maps of up to 2x2 below 1,024
     // pixels, whose taps mostly fall outside (512 -> 512 at B=128: 54 against
