@@ -111,7 +111,7 @@ int vdttfs_bucketize(vdttfs_ctx* ctx, const float* d_in, int64_t n_cols, int c_i
  * neuron never fires), NHWC with c_out fastest.  This is the reference-layout
  * export path, kept for bit-exact checks of caller-made buckets: the entries
  * are listed in context scratch and streamed a pixel per wave; past 25 taps,
- * 1024 outputs or 65535 weight rows, without memory for the lists, or under
+ * 1024 outputs or 16384 weight rows, without memory for the lists, or under
  * stream capture where no earlier call has made the scratch large enough, one
  * thread per neuron walks them.  vdttfs_layer_forward takes
  * the dense map.  Buckets are expected from this context's constants; events

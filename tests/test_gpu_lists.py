@@ -32,6 +32,23 @@ SHAPES = [
     ("t200-fc-4100-700", 200, 0, False, True, 3, 1, 1, 4100, 700, 1),
     ("t65-fc-3-1", 65, 0, True, True, 5, 1, 1, 3, 1, 1),
 ]
+# either side of the lengths up to which a layer takes the lists
+LENGTHS = [
+    ("t80-fc-2048-70", 80, 0, True, True, 31, 1, 1, 2048, 70, 1),
+    ("t80-fc-2049-70", 80, 0, True, True, 31, 1, 1, 2049, 70, 1),
+    ("t80-fc-4096-70", 80, 0, True, True, 33, 1, 1, 4096, 70, 1),
+    ("t80-fc-4097-70", 80, 0, True, True, 33, 1, 1, 4097, 70, 1),
+    ("t80-conv3-256-140", 80, 0, True, False, 2, 5, 4, 256, 140, 3),
+    ("t80-conv3-257-140", 80, 0, True, False, 2, 5, 4, 257, 140, 3),
+    ("t80-conv5-80-20", 80, 0, True, False, 1, 5, 4, 80, 20, 5),
+    ("t80-conv5-81-20", 80, 0, True, False, 1, 5, 4, 81, 20, 5),
+]
+
+
+@pytest.mark.parametrize("kind", ["random", "dense"])
+@pytest.mark.parametrize("shape", LENGTHS, ids=[s[0] for s in LENGTHS])
+def test_lists_lengths(gpu_ctx_factory, shape, kind):
+    test_lists_match_oracle(gpu_ctx_factory, shape, kind)
 
 
 @pytest.mark.parametrize("kind", ["random", "silent", "bin0", "one-late-bin", "last-bin", "dense", "fractional"])

@@ -41,7 +41,7 @@ SHAPES = [
 # k_gemm0's tile of a wave (pixels x c_out), then a shape that takes it
 TILES = [
     ((16, 16), ("t64-conv5-5-33-small", 64, 32, True, False, 7, 6, 7, 5, 33, 5)),
-    ((16, 16), ("t128-conv3-36-131", 128, 64, True, False, 2, 6, 7, 36, 131, 3)),         # two bin blocks
+    ((16, 16), ("t128-conv3-65-131", 128, 64, True, False, 2, 6, 7, 65, 131, 3)),         # two bin blocks
     ((32, 32), ("t64-conv5-5-33", 64, 32, True, False, 147, 13, 11, 5, 33, 5)),
     ((32, 32), ("t64-conv5-3-34", 64, 32, False, False, 149, 13, 14, 3, 34, 5)),
     ((32, 32), ("t64-conv5-5-33-pos", 64, 32, True, False, 353, 5, 7, 5, 33, 5)),         # (position, image) rows
@@ -128,8 +128,10 @@ def tile_of(shape):
     tiles = -(-pix // 32) * -(-C_out // 32)
     if C_out < 32 or 4 * tfs < T or T > 128:
         return None
+    if taps > 9 and nel > 3000:
+        return None
     if T > 64:
-        if nel <= 300:
+        if nel <= 300 or taps == 1 or (nel <= 576 and pix <= 1024):
             return None
     elif taps > 9:
         if nel < 4:
@@ -151,8 +153,16 @@ LINES = [  # either side of the lines that the split is chosen by
     (None, ("t64-conv3-20-70-767", 64, 32, True, False, 15, 34, 16, 20, 70, 3)),
     (None, ("t64-conv3-20-70-early", 64, 31, True, False, 16, 32, 16, 20, 70, 3)),
     ((32, 64), ("t64-conv3-20-66-early", 64, 31, True, False, 45, 31, 32, 20, 66, 3)),
-    (None, ("t80-conv5-12-40", 80, 40, True, False, 2, 9, 7, 12, 40, 5)),  # 300 elements: column lists
-    ((16, 16), ("t80-conv1-301-40", 80, 40, True, False, 3, 9, 7, 301, 40, 1)),
+    # past 64 steps short fields and single taps take the column lists
+    (None, ("t80-conv5-12-40", 80, 40, True, False, 17, 9, 7, 12, 40, 5)),
+    ((16, 16), ("t80-conv5-13-40", 80, 40, True, False, 17, 9, 7, 13, 40, 5)),
+    (None, ("t80-conv3-64-40", 80, 40, True, False, 3, 9, 7, 64, 40, 3)),
+    ((16, 16), ("t80-conv3-65-40", 80, 40, True, False, 3, 9, 7, 65, 40, 3)),
+    (None, ("t80-conv1-601-40", 80, 40, True, False, 3, 9, 7, 601, 40, 1)),
+    # long fields of many taps the merged lists
+    ((16, 16), ("t64-conv5-120-140", 64, 32, True, False, 2, 6, 5, 120, 140, 5)),
+    (None, ("t64-conv5-121-40", 64, 32, True, False, 2, 6, 5, 121, 40, 5)),
+    (None, ("t80-conv5-121-40", 80, 40, True, False, 2, 6, 5, 121, 40, 5)),
     (None, ("t64-conv3-15-99", 64, 32, True, False, 16, 32, 16, 15, 99, 3)),
     ((32, 32), ("t64-conv3-16-99", 64, 32, True, False, 16, 32, 16, 16, 99, 3)),
 ]

@@ -1013,15 +1013,23 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
     // Three launches and the element chain of k_gemm0 (32 cycles an element,
     // 8 in 16x16 tiles) need work to hide under.  Where the fused kernels do
     // not serve (T > 64, or more than 9 taps: bucketize or dense merge and a
-    // stream) that is any layer of a few inputs past nine taps.
+    // stream) that is any layer of a few inputs past nine taps, until the list
+    // comes in many windows, each of which reads it from its start (times as
+    // fast as merged lists at densities 0.1 / 0.3 / 0.7: 64 outputs, 64 pixels,
+    // 2,500 elements 1.21 / 1.34 / 1.15, 3,500 1.13 / 1.27 / 0.90, 5,000 1.02 /
+    // 0.98 / 0.72; 200 outputs, 4,096 pixels, 2,500 0.87 / 1.14 / 1.33, 5,000
+    // 0.72 / 1.03 / 1.25).
+    if (taps > 9 && K > 3000) return false;
     if (T <= 64 && taps > 9) return K >= 4;
     // Past 64 steps the lists of every bin (two launches) are there as well and
     // finish first in short fields, where the split even lost to the kernels
     // before it (3x3, C_in 3, 64 outputs, T = 80, 1,024 pixels, us at densities
     // 0.1 / 0.7: dense merge and stream 11.9 / 16.0, split 14.9 / 15.4, lists
     // 8.4 / 9.2; times as fast as the split: 72 elements 1.75 / 1.6, 171 1.7 /
-    // 1.35, 300 1.9 / 1.2, 576 1.7 / 1.06 there and 1.5 / 0.8 at 16K pixels).
-    if (T > 64) return K > 300;
+    // 1.35, 300 1.9 / 1.2, 576 1.7 / 1.06 there and 1.5 / 0.8 at 16K pixels), and
+    // at one tap outside networks (1,500 elements, 128 outputs, 1,024 pixels:
+    // split 0.92 / 1.61 times the speed of merged lists, lists 1.59 / 1.38).
+    if (T > 64) return K > 300 && (net || (taps > 1 && (K > 576 || pix > 1024)));
     // Against the fused kernels: FC layers keep them (VGG-16's 512 -> 512 at
     // B=256: 28 against 34 us), and so do maps of up to 2x2 below 1,024
     // pixels, whose taps mostly fall outside (512 -> 512 at B=128: 54 against
@@ -1087,7 +1095,22 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
 // the register and narrow kernels do (batch 1024: conv1 145 against 567 us,
 // conv2 169 against 169).  Each group of four c_out blocks rebuilds a pixel's
 // list, so layers past 1024 outputs keep the merged lists.
-bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return ctx->c.T > 64 && lists_fit(ctx, s); }
+//
+// So do long lists: one past `cap` entries is read from its start for every
+// window of it, where the merged lists are read once.  Times as fast as those,
+// T = 80: FC to 128 outputs, 32 images, densities 0.05 / 0.3 / 1: 2,000 inputs
+// 1.34 / 1.47 / 1.16, 4,096 1.13 / 1.21 / 0.77, 8,192 1.01 / 0.91 / 0.67, 16,384
+// 0.83 / 0.86 / 0.42; one image to 10 outputs 2,000 1.37 / 1.10 / 0.88, 4,096
+// 1.03 / 0.92 / 0.58; 3x3, 512 channels, 1,024 pixels, densities 0.1 / 0.7: 128
+// outputs 1.84 / 1.11, 512 outputs 1.20 / 0.65; 5x5, 200 channels (each entry's
+// tap is found among 25): 32 outputs 1.65 / 0.34, 128 1.64 / 0.50.
+bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
+    if (ctx->c.T <= 64 || !lists_fit(ctx, s)) return false;
+    const int taps = s.is_fc ? 1 : s.K_h * s.K_w, K = taps * s.C_in;
+    if (taps > 9) return K <= 2000;
+    if (taps > 1 && s.C_out > 128) return K <= 2304;
+    return K <= (split_pix(s) < 32 ? 2048 : 4096);
+}
 
 int split_choice(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
     // (up to 64 steps fields of at most 32 elements have a plan of their own)
@@ -1097,7 +1120,12 @@ int split_choice(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
     return lists_ok(ctx, s) ? kSplitLists : 0;
 }
 
-bool ref_lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) { return lists_fit(ctx, s); }
+// Over the reference's buckets the other way is the loop nest, which the lists
+// beat up to 16,384 elements whatever arrives (all inputs active, 32 columns, 10
+// outputs: 8,192 3.2 times as fast, 16,384 1.9, 32,768 1.0; one column 1.3, 0.7).
+bool ref_lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
+    return lists_fit(ctx, s) && (s.is_fc ? 1 : s.K_h * s.K_w) * s.C_in <= 16384;
+}
 
 namespace {
 
