@@ -42,9 +42,11 @@ stream, the dominant kernel family):
   so it exceeds the HBM peak.
 * roofline.gathered -- the weight bytes the stream kernels gather per
   integrated synapse (4 B per event under the per-bin exit the kernels run,
-  E_bin) over the same time, against the gather roof that
-  vdttfs_probe_gather measures live on the same GPU (weights resident in
-  one XCD's L2): this is the ceiling the stream kernels are bound by.
+  E_bin) over the time of the layers that run on them, against the gather
+  roof that vdttfs_probe_gather measures live on the same GPU (weights
+  resident in one XCD's L2): this is the ceiling the stream kernels are bound
+  by.  Layers on the split integrator (bin 0 on the matrix cores) or the pixel
+  kernel (weights in LDS) are not in it.
 """
 from __future__ import annotations
 
@@ -329,22 +331,27 @@ def work_table(ctx, net, w, B, d_img, counts, layer_ms, roofs, tr):
                 l.C_out, 1 if fc else l.K_h, 1 if fc else l.K_w, ph, pw, fc, tfs, T)
             ms = float(layer_ms[i])
             path, gather, ppw = net.get_plan(i)
+            route = ["plan", "split", "lists", "pixel"][net.get_route(i)]
+            # the split sums bin 0 on the matrix cores and the pixel kernel reads
+            # its weights from LDS: E_bin says nothing about their gathers
+            gathers = route in ("plan", "lists")
             # dword gathers: one c_out per lane outside the fused path (k_stream,
-            # k_stream_narrow, k_conv_small); the fused path (k_stream_quad)
-            # and gathers 2 and 4 load dwordx4
-            roof = roofs[1] if gather == 1 and path != 3 else roofs[4]
+            # k_stream_narrow, k_conv_small); the fused path (k_stream_quad),
+            # the lists (k_late) and gathers 2 and 4 load dwordx4
+            roof = roofs[1] if gather == 1 and path != 3 and route == "plan" else roofs[4]
             gb = 4.0 * float(ebin[i])
             row = {"layer": i, "kind": "fc" if fc else "conv",
                    "shape": f"{l.C_in}->{l.C_out} @ {l.H_in}x{l.W_in}" + ("" if fc else f", {l.K_h}x{l.K_w}"),
+                   "route": route,
                    "plan": {"path": ["auto", "bins", "dense", "fused", "reg", "window"][path], "gather": gather,
-                            "ppw": ppw},
+                            "ppw": ppw} if route == "plan" else None,
                    "ms": ms, "eproc": int(eproc[i]), "ebin": int(ebin[i]), "e_noee": e_noee,
                    "skip_rate": 1.0 - float(eproc[i]) / max(1, e_noee),
                    "n_ev": int(n_ev[i]), "n_ev_host_equal": nev == int(n_ev[i]),
                    "in_density": nev / float(x.size), "out_fired": float(np.mean(out < 9999.0)),
-                   "gathered_GBps": gb / (ms * 1e-3) / 1e9,
-                   "gather_roof_GBps": roof["GBps"],
-                   "gather_frac": gb / (ms * 1e-3) / 1e9 / roof["GBps"],
+                   "gathered_GBps": gb / (ms * 1e-3) / 1e9 if gathers else None,
+                   "gather_roof_GBps": roof["GBps"] if gathers else None,
+                   "gather_frac": gb / (ms * 1e-3) / 1e9 / roof["GBps"] if gathers else None,
                    "algorithmic_hbm_bytes": hbm_compulsory_bytes(l, B),
                    "b_int_bytes": b_int_bytes(l, B, int(eproc[i]), int(n_ev[i]), int(n_cols[i]),
                                               w.consts.num_chunks + 1)}
@@ -511,9 +518,12 @@ def bench_ttfs(args) -> int:
     integ_s = integ_ms_step * 1e-3
     alg = sum(r["algorithmic_hbm_bytes"] for r in rows)
     b_int = sum(r["b_int_bytes"] for r in rows)
-    gathered = sum(4.0 * r["ebin"] for r in rows)
-    # time the layers would take at their gather roof, over the time they took
-    t_roof = sum(4.0 * r["ebin"] / (r["gather_roof_GBps"] * 1e9) for r in rows)
+    # the layers whose kernels gather a weight row per event: their bytes, their
+    # time, and the time they would take at their gather roof
+    gat = [r for r in rows if r["gather_roof_GBps"]]
+    gathered = sum(4.0 * r["ebin"] for r in gat)
+    gather_s = sum(r["ms"] for r in gat) * 1e-3
+    t_roof = sum(4.0 * r["ebin"] / (r["gather_roof_GBps"] * 1e9) for r in gat)
     dense = 0
     for l in w.layers:
         if l.kind == 0:
@@ -579,14 +589,16 @@ def bench_ttfs(args) -> int:
             },
             "gathered": {
                 "bytes_per_step": gathered,
-                "achieved_GBps": gathered / integ_s / 1e9,
+                "layers": [r["layer"] for r in gat],
+                "achieved_GBps": gathered / gather_s / 1e9 if gat else None,
                 "roof_GBps_dword": roofs[1]["GBps"],
                 "roof_GBps_dwordx4": roofs[4]["GBps"],
-                "frac": t_roof / integ_s,
-                "model": "4 B per integrated synapse under the per-bin exit the kernels run (E_bin); roof = "
-                         "vdttfs_probe_gather with weights in one XCD's L2, dword rows for layers gathering one "
-                         "c_out per lane outside the fused path, dwordx4 rows for the others; frac = (time at "
-                         "each layer's roof) / (integrator time)",
+                "frac": t_roof / gather_s if gat else None,
+                "model": "4 B per integrated synapse under the per-bin exit the kernels run (E_bin), over the layers "
+                         "that gather every event's weights (not the split, whose bin 0 is a matrix product, nor the "
+                         "pixel kernel); roof = vdttfs_probe_gather with weights in one XCD's L2, dword rows for "
+                         "layers gathering one c_out per lane outside the fused path, dwordx4 rows for the others; "
+                         "frac = (time at each layer's roof) / (those layers' time)",
                 "probe": roofs,
             },
         },

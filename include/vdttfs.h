@@ -347,11 +347,11 @@ int vdttfs_net_set_windows(vdttfs_net* net, const int32_t* windows, int n_layers
  * (> 25 taps) take the generic integrator (path BINS, gather and ppw 0).
  * Pool and vmem layers have no plan.  set_plan(NULL) restores the built-in
  * choice; an unsupported request fails with VDTTFS_E_UNSUPPORTED and leaves
- * the layer's plan unchanged.  Where no field is asked for, a layer whose fire
- * start is a quarter of its window or more may run on the split kernels (bin 0
- * on the matrix cores), which have no plan fields: get_plan then names the plan
- * that its counting forwards, and forwards with a pool fused into it, take.  get_plan returns the resolved plan the next
- * forward uses. */
+ * the layer's plan unchanged.  get_plan returns the resolved plan.  Where no
+ * field is asked for, a layer may run on kernels that have no plan fields
+ * (get_route below); get_plan then names the plan that its counting forwards,
+ * and forwards with a pool fused into it, take.  Setting that plan is not the
+ * same as leaving the layer built in. */
 #define VDTTFS_PATH_AUTO   0
 #define VDTTFS_PATH_BINS   1
 #define VDTTFS_PATH_DENSE  2
@@ -363,6 +363,15 @@ typedef struct vdttfs_layer_plan {
 } vdttfs_layer_plan;
 int vdttfs_net_set_plan(vdttfs_net* net, int layer, const vdttfs_layer_plan* plan);
 int vdttfs_net_get_plan(vdttfs_net* net, int layer, vdttfs_layer_plan* out);
+/* The kernels that the layer's next forward without counters and without a pool
+ * fused into it runs on: those of its plan, the split integrator (bin 0 on the
+ * matrix cores, later bins from column lists), the column lists over every bin,
+ * or a pixel per lane (its weights from LDS, no lists). */
+#define VDTTFS_ROUTE_PLAN  0
+#define VDTTFS_ROUTE_SPLIT 1
+#define VDTTFS_ROUTE_LISTS 2
+#define VDTTFS_ROUTE_PIXEL 3
+int vdttfs_net_get_route(vdttfs_net* net, int layer, int32_t* out);
 /* Per-layer event time (bucketize + integrator launches, ms) summed over the
  * timed forwards since the last read (timing enabled with
  * vdttfs_net_set_timing); ms has n_layers entries, pools and vmem read 0.

@@ -155,6 +155,49 @@ def test_every_plan_matches_oracle_lenet(gpu_ctx_factory):
     assert n[0] == 3 and n[6] == 2  # FC 84 -> 10: the narrow bins path and the shared-list kernel
 
 
+def test_routes_follow_sizes_and_plans(gpu_ctx_factory):
+    """get_route on VGG-16: the split where the layers are large or long, the
+    plan's kernels on the 2x2 maps, the FC layer and pools, on the 4x4 layers
+    (their weights past an XCD's L2) between 49 and 383 pixels, and wherever a
+    plan is set; LeNet-5's convolutions a pixel per lane where it pays; lists
+    past 64 steps.  Every network equals the oracle."""
+    PLAN, SPLIT, LISTS, PIXEL = vdttfs.ROUTE_PLAN, vdttfs.ROUTE_SPLIT, vdttfs.ROUTE_LISTS, vdttfs.ROUTE_PIXEL
+    split = (6, 7, 8)
+    wide = (10, 11, 12)
+    for B, exp in ((3, split + wide), (4, (1,) + split), (23, (0, 1, 3, 4) + split), (24, (0, 1, 3, 4) + split + wide)):
+        say(f"routes: VGG-16 B={B}")
+        w = models.vgg16()
+        net = make_net(gpu_ctx_factory(w.consts), w, B)
+        try:
+            for i in range(len(w.layers)):
+                assert net.get_route(i) in (PLAN, SPLIT)
+            got = tuple(i for i in range(len(w.layers)) if net.get_route(i) == SPLIT)
+            assert set(wide) <= set(got) if set(wide) <= set(exp) else not set(wide) & set(got), got
+            assert set(split) <= set(got) and not set(got) & {2, 14, 15, 16, 18, 19}, got
+            net.set_plan(6, *net.get_plan(6))
+            assert net.get_route(6) == PLAN  # the named plan is not the built-in choice
+            net.set_plan(6)
+            assert net.get_route(6) == SPLIT
+            img = models.images_for(w, B)
+            net.forward(net.ctx.to_device(img))
+            net.ctx.synchronize()
+            ref = oracle_ref(w, B, img)["outs"]
+            for i in range(len(w.layers)):
+                if w.layers[i].kind != vdttfs.LAYER_VMEM:
+                    np.testing.assert_array_equal(net.layer_output(i).reshape(-1), ref[i].reshape(-1), err_msg=str(i))
+        finally:
+            net.close()
+    for T, B, exp in ((64, 32, {0: PIXEL, 2: PLAN, 4: PLAN, 6: PLAN}), (64, 1024, {0: PIXEL, 2: PIXEL, 4: PLAN}),
+                      (80, 8, {0: PIXEL, 2: LISTS, 4: LISTS, 6: LISTS})):
+        say(f"routes: LeNet-5 T={T} B={B}")
+        w = models.lenet5(T=T)
+        net = make_net(gpu_ctx_factory(w.consts), w, B)
+        try:
+            assert {i: net.get_route(i) for i in exp} == exp
+        finally:
+            net.close()
+
+
 def test_tuner_lenet(gpu_ctx_factory):
     say("tuner: LeNet-5 B=64 Delta sweep and plan sweep")
     w = models.lenet5()

@@ -194,6 +194,14 @@ class WindowScope {
     int T_, NC_, OS_;
 };
 
+// Whether a forward without counters and without a fused pool leaves the named
+// plan for the built-in choice of layers with a late fire start, a long window
+// or few outputs.  Their scratch is the merged lists' buffer, sized for both at
+// creation where there was the memory.
+bool takes_split(const vdttfs_net* net, const IntegShape& s, const LaunchPlan& p) {
+    return p.split && (p.split == kSplitPixel || split_scratch_bytes(s) <= net->list_bytes);
+}
+
 // counters: nullable; when set, per-layer instrumented run
 int forward_impl(vdttfs_net* net, const float* d_img, int32_t* d_pred, uint64_t* eproc,
                  uint64_t* ebin, uint64_t* n_ev, uint64_t* n_cols) {
@@ -255,11 +263,7 @@ int forward_impl(vdttfs_net* net, const float* d_img, int32_t* d_pred, uint64_t*
             // and in a counting forward for its retained-event count
             LaunchPlan plan;
             VD_TRY(resolve_plan(ctx, s, l.plan, &plan, /*net=*/true));
-            // the built-in choice of layers with a late fire start or a long
-            // window; its scratch is the merged lists' (sized for both at
-            // creation, where there was the memory)
-            const bool split = plan.split && !count && !fuse &&
-                               (plan.split == kSplitPixel || split_scratch_bytes(s) <= net->list_bytes);
+            const bool split = !count && !fuse && takes_split(net, s, plan);
             const bool dense = split || plan_from_dense(ctx, s, plan, count);
             TimedPair tb{}, ti{};
             tb.layer = ti.layer = (int)i;
@@ -688,6 +692,25 @@ int vdttfs_net_get_plan(vdttfs_net* net, int layer, vdttfs_layer_plan* out) {
     LaunchPlan p;
     VD_TRY(resolve_plan(ctx, integ_shape(net, l), l.plan, &p));
     *out = vdttfs_layer_plan{p.path, p.gather, p.ppw};
+    return VDTTFS_OK;
+}
+
+int vdttfs_net_get_route(vdttfs_net* net, int layer, int32_t* out) {
+    if (!net || !out || layer < 0 || layer >= (int)net->L.size())
+        return set_error(VDTTFS_E_INVALID, "net_get_route: bad argument");
+    const NetLayer& l = net->L[layer];
+    *out = VDTTFS_ROUTE_PLAN;
+    if (l.d.kind != VDTTFS_LAYER_CONV && l.d.kind != VDTTFS_LAYER_FC) return VDTTFS_OK;
+    vdttfs_ctx* ctx = net->ctx;
+    WindowScope window(ctx, l.window);
+    const IntegShape s = integ_shape(net, l);
+    LaunchPlan p;
+    VD_TRY(resolve_plan(ctx, s, l.plan, &p, /*net=*/true));
+    if (takes_split(net, s, p))
+        *out = p.split == kSplitDense ? VDTTFS_ROUTE_SPLIT
+                                      : (p.split == kSplitLists ? VDTTFS_ROUTE_LISTS : VDTTFS_ROUTE_PIXEL);
+    else if (p.path == VDTTFS_PATH_REG && conv_px_ok(ctx->c.T, s))  // launch_conv_small hands over
+        *out = VDTTFS_ROUTE_PIXEL;
     return VDTTFS_OK;
 }
 

@@ -18,7 +18,8 @@ from ._lib import (Consts, CulifLayer, LayerDesc, VdttfsError, check, lib, INF_T
                    LAYER_CONV, LAYER_FC, LAYER_POOL, LAYER_VMEM, ENCODE_LINEAR, ENCODE_LOG, ENCODE_TIMES,
                    READOUT_ARGMIN, READOUT_ARGMAX, CULIF_RAW_CONV, CULIF_CONV, CULIF_POOL,
                    CULIF_FC_REC, CULIF_FC, STEP_T1, STEP_T2, STEP_T3, LayerPlan, PATH_AUTO, PATH_BINS, PATH_DENSE,
-                   PATH_FUSED, PATH_REG, PATH_WINDOW, POOL_FUSE_OFF, POOL_FUSE_ALL, POOL_FUSE_AUTO)
+                   PATH_FUSED, PATH_REG, PATH_WINDOW, ROUTE_PLAN, ROUTE_SPLIT, ROUTE_LISTS,
+                   ROUTE_PIXEL, POOL_FUSE_OFF, POOL_FUSE_ALL, POOL_FUSE_AUTO)
 
 
 def _ptr(a: np.ndarray) -> C.c_void_p:
@@ -371,10 +372,18 @@ class Net:
         check(lib().vdttfs_net_set_plan(self.handle, layer, C.byref(pl)))
 
     def get_plan(self, layer: int) -> tuple:
-        """(path, gather, ppw) the next forward uses for the layer."""
+        """(path, gather, ppw) of the layer's plan; a built-in layer may run on
+        kernels outside it (get_route)."""
         pl = LayerPlan()
         check(lib().vdttfs_net_get_plan(self.handle, layer, C.byref(pl)))
         return pl.path, pl.gather, pl.ppw
+
+    def get_route(self, layer: int) -> int:
+        """The kernels of the layer's next forward (vdttfs_net_get_route):
+        ROUTE_PLAN, _SPLIT, _LISTS or _PIXEL."""
+        r = C.c_int32()
+        check(lib().vdttfs_net_get_route(self.handle, layer, C.byref(r)))
+        return r.value
 
     def read_layer_timing(self) -> np.ndarray:
         """Per-layer event ms since the last read (timing must be enabled)."""
