@@ -209,6 +209,8 @@ def test_tuner_lenet(gpu_ctx_factory):
     assert all(r["ms_per_batch"] > 0 for r in rows)
     r = tune.tune_plans(w, img, B, reps=1, rounds=1)
     assert r["tuned_identical"]
+    assert all(p is None or "builtin" not in p or p["builtin"] for p in r["plans"])
+    assert all(L["candidates"][0]["plan"]["builtin"] for L in r["layers"])
     # LeNet-5's pools feed the dense-merge conv and a flattened FC: no build takes them
     assert set(r["pool_fusion"]["modes"]) == {"off", "auto", "all"}
     assert all(v["identical"] and v["ms"] > 0 for v in r["pool_fusion"]["modes"].values())

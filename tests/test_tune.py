@@ -40,6 +40,34 @@ def test_load_plans_checks_workload(tmp_path):
         tune.load_pool_fusion(str(f), w, 64)
 
 
+class FakeNet:
+    """The tuner's view of a network with one integrating layer: a time per
+    plan, None being the built-in choice."""
+
+    def __init__(self, layers, ms):
+        self.layers, self.ms, self.plans = layers, ms, {}
+
+    def set_plan(self, layer, *plan):
+        self.plans[layer] = plan or None
+        if plan and plan not in self.ms:
+            raise vdttfs.VdttfsError(-6, "plan")
+
+
+@pytest.mark.parametrize("builtin_ms,wins", [(1.0, True), (2.0, True), (3.0, False)])
+def test_builtin_choice_is_a_candidate(builtin_ms, wins):
+    """A layer whose built-in time is the lowest keeps the built-in choice,
+    whose kernels may have no plan of their own."""
+    named = [{"plan": {"path": "fused", "gather": 2, "ppw": 1}, "ms": 2.0, "identical": True},
+             {"plan": {"path": "bins", "gather": 4, "ppw": 2}, "ms": 0.5, "identical": False}]
+    auto = {"plan": {"path": "fused", "gather": 2, "ppw": 1, "builtin": True}, "ms": builtin_ms, "identical": True}
+    best = tune.best_candidate([auto] + named)
+    assert (best is auto) == wins
+    net = FakeNet([None], {(vdttfs.PATH_FUSED, 2, 1): 2.0})
+    tune.apply_plans(net, [best["plan"]])
+    assert net.plans[0] == (None if wins else (vdttfs.PATH_FUSED, 2, 1))
+    assert tune.best_candidate([named[1]]) is None
+
+
 def test_committed_vgg_plans_fit_the_benchmark():
     """configs/plans_vgg16_b256.json (tuned on MI355X, bench.py --plans) names
     a plan for exactly the integrating layers of the benchmark network."""

@@ -15,7 +15,12 @@ c_out a lane gathers per event (1, 2 events per load, or 4), and how many
 output pixels a wave integrates.  The tuner sweeps them per layer with the
 reference's procedure -- minimum of three timed rounds, outputs compared bit
 for bit with the built-in choice -- and reports the best plan per layer and
-the whole forward under the tuned plans; then, under those plans, which 2x2
+the whole forward under the tuned plans.  The built-in choice is a candidate
+like the others: it may run kernels that have no plan fields (the split
+integrator, the column lists, a pixel per lane), and a plan record that says
+"builtin" leaves the layer to it, its fields being those of the named plan
+that counting forwards take.  Where the whole forward is no faster under the
+tuned plans, every layer stays built in.  Then, under those plans, which 2x2
 pools run inside the next layer's list build (vdttfs_net_set_pool_fusion:
 off, auto or all), timed on the whole forward.
 
@@ -118,31 +123,32 @@ def tune_plans(w, img, B, reps=3, rounds=3):
             base = _min_round_ms(ctx, net, x, d_pred, reps, rounds, True)
             ref = [net.layer_output(i) for i in range(n)]
             fwd_auto = float(_min_round_ms(ctx, net, x, d_pred, reps, rounds, False))
-            rows, best_plans = [], list(auto_plans)
+            builtin = [dict(_plan_dict(p), builtin=True) if l.kind in (core.LAYER_CONV, core.LAYER_FC) else None
+                       for l, p in zip(w.layers, auto_plans)]
+            rows, plans = [], list(builtin)
             for i, l in enumerate(w.layers):
                 if l.kind not in (core.LAYER_CONV, core.LAYER_FC):
                     continue
                 cands = []
-                for plan in candidates(net, i):
-                    net.set_plan(i, *plan)
+                for plan in [None] + candidates(net, i):
+                    net.set_plan(i, *(plan or ()))
                     ms = float(_min_round_ms(ctx, net, x, d_pred, reps, rounds, True)[i])
                     same = bool(np.array_equal(net.layer_output(i), ref[i]))
-                    cands.append({"plan": _plan_dict(plan), "ms": ms, "identical": same})
+                    cands.append({"plan": _plan_dict(plan) if plan else builtin[i], "ms": ms, "identical": same})
                 net.set_plan(i)
-                ok = [c for c in cands if c["identical"]]
-                best = min(ok, key=lambda c: c["ms"]) if ok else None
+                best = best_candidate(cands)
                 if best is not None:
-                    p = best["plan"]
-                    best_plans[i] = (_path_id(p["path"]), p["gather"], p["ppw"])
+                    plans[i] = best["plan"]
                 rows.append({"layer": i, "kind": "conv" if l.kind == core.LAYER_CONV else "fc",
                              "shape": [l.H_in, l.W_in, l.C_in, l.C_out, l.K_h, l.K_w],
                              "auto": {"plan": _plan_dict(auto_plans[i]), "ms": float(base[i])},
                              "best": best, "candidates": cands,
                              "all_identical": all(c["identical"] for c in cands)})
-            for i, p in enumerate(best_plans):
-                if w.layers[i].kind in (core.LAYER_CONV, core.LAYER_FC):
-                    net.set_plan(i, *p)
+            apply_plans(net, plans)
             fwd_tuned = float(_min_round_ms(ctx, net, x, d_pred, reps, rounds, False))
+            if fwd_tuned >= fwd_auto:
+                plans = list(builtin)
+                apply_plans(net, plans)
             tuned_same = all(np.array_equal(net.layer_output(i), ref[i]) for i in range(n))
             # pool fusion under the tuned plans: the whole forward per mode
             # (a fused pool's map is written when layer_output asks for it)
@@ -161,8 +167,14 @@ def tune_plans(w, img, B, reps=3, rounds=3):
             net.close()
     return {"layers": rows, "forward_ms": {"auto": fwd_auto, "tuned": fwd_tuned},
             "tuned_identical": tuned_same, "pool_fusion": {"modes": fusion, "best": best_fusion},
-            "plans": [_plan_dict(p) if w.layers[i].kind in (core.LAYER_CONV, core.LAYER_FC) else None
-                      for i, p in enumerate(best_plans)]}
+            "plans": plans}
+
+
+def best_candidate(cands):
+    """The fastest candidate whose outputs equal the built-in choice's (on a
+    tie the built-in choice), or None."""
+    ok = [c for c in cands if c["identical"]]
+    return min(ok, key=lambda c: (c["ms"], not c["plan"].get("builtin", False))) if ok else None
 
 
 def _plan_dict(p):
@@ -174,11 +186,14 @@ def _path_id(name):
 
 
 def apply_plans(net, plans):
-    """Sets the plans of a tune result ("plans": one dict or None per layer)."""
+    """Sets the plans of a tune result ("plans": one dict or None per layer;
+    "builtin" restores the layer's built-in choice)."""
     if len(plans) != len(net.layers):
         raise ValueError(f"{len(plans)} plans for {len(net.layers)} layers")
     for i, p in enumerate(plans):
-        if p is not None:
+        if p is not None and p.get("builtin"):
+            net.set_plan(i)
+        elif p is not None:
             net.set_plan(i, _path_id(p["path"]), p["gather"], p["ppw"])
 
 
