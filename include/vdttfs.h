@@ -140,10 +140,13 @@ int vdttfs_layer_forward(vdttfs_ctx* ctx, float* d_out, const float* d_in,
 /* ---- the layer path without device allocation ------------------------- */
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc): the same kernels and results as vdttfs_layer_forward
- * (without the work counters), with the layer's merged lists and bucket
- * scratch in a 64 MiB device buffer that the library holds per GPU until the
- * process ends, instead of context scratch grown with hipMalloc.  The call
+ * forbid hipMalloc): the same results as vdttfs_layer_forward (without the work
+ * counters) from the kernels of the layer's named plan (vdttfs_layer_plan, all
+ * fields 0), with its merged lists and bucket scratch in a 64 MiB device buffer
+ * that the library holds per GPU until the process ends, instead of context
+ * scratch grown with hipMalloc.  The split integrator and the column lists,
+ * which layer_forward runs where they are faster, are not taken here: VGG-16's
+ * layers at batch 256 take about twice as long.  The call
  * allocates and frees nothing.  A layer whose scratch exceeds 64 MiB fails
  * with VDTTFS_E_UNSUPPORTED (the LDS-list and register paths need none: every
  * layer of the VGG-16 and LeNet-5 configurations runs; a layer on the
@@ -384,9 +387,11 @@ int vdttfs_net_read_timing(vdttfs_net* net, double* integ_ms, int64_t* integ_lau
  *      denominator, T1S = task1_lenet_mnist/stepbystep_cuda/
  *      snn_mnist_stepbystep.cu, T2S = task2_vgg16_cifar10/stepbystep_cuda/
  *      bench_vgg_timedriven_baseline.cu ------------------------------------ */
-/* Every global step launches every layer: each neuron sums the weights of
- * the inputs that spike at that step and fires once on the decaying
- * threshold.  mode VDTTFS_STEP_T1 (T1S:47-103, 222-244): all layers share
+/* At every global step each neuron sums the weights of the inputs that spike
+ * at that step and fires once on the decaying threshold.  T1 and T2 run layer by
+ * layer, each over all steps in one launch (a neuron scans its field once, not
+ * once a step), so they give the reference's results and not its cost; T3
+ * launches every layer at every step.  mode VDTTFS_STEP_T1 (T1S:47-103, 222-244): all layers share
  * the step, V = fma(sum w, kv(t), V), the last layer's first spike is the
  * output (argmin readout), T steps.  mode VDTTFS_STEP_T2 (T2S:53-200,
  * 329-352): weighted layer d integrates at t - (d-1)*tfs in [0, T) with

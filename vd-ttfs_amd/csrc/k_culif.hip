@@ -285,10 +285,12 @@ __global__ __launch_bounds__(256) void k_culif_event_masks(MaskArgs a) {
 // an SGPR lane mask and each lane counts the steps it has lived through, which
 // is its spike step once it fires.
 //
-// Bound by the matrix unit (128 cycles per pair of taps and 32 steps) and the
-// neuron steps.  Visiting the set taps one by one (a scalar bit scan and an
-// indexed register add each) took 1,370 us on CuLIF-7's conv1 (B=64, 128x128,
-// 2 -> 64, T=64) where this takes 849.
+// No unit is busy half the time: the matrix unit 26% (128 cycles per pair of
+// taps and 32 steps), vector issue 42% (the neuron steps), scalar issue 45% (the
+// masks); they follow each other in a wave, and 13 waves a CU do not fill the
+// gaps.  Visiting the set taps one by one (a scalar bit scan and an indexed
+// register add each) took 1,370 us on CuLIF-7's conv1 (B=64, 128x128, 2 -> 64,
+// T=64) where this takes 849.
 template <int NK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_culif_conv1_mask(
     RawArgs a, const uint64_t* __restrict__ mask, const uint32_t* __restrict__ nonbin, int nblk, int ppw) {

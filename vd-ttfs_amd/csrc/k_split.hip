@@ -38,7 +38,8 @@ constexpr int kLateMaxWaves = 4;
 constexpr int kLateKeep = 2;      // chunks per wave kept in registers between the two passes
 
 // ---------------------------------------------------------------------------
-// What k_late needs of a layer's thresholds, prepared once per call by k_split.
+// What k_late needs of a layer's thresholds, prepared once per call by the
+// kernel that writes its lists (k_split or k_ref_lists).
 struct LateThr {
     float th[kSplitMaxT];  // theta where a spike may occur (t >= t_min, theta >= 1e-5), else NaN
     // Where those bins are one run [lo, hi) with non-increasing thresholds
@@ -52,43 +53,43 @@ struct LateThr {
 // A workgroup of 256 threads fills *thr.
 __device__ inline void prepare_thresholds(const float* theta, int T, int t_min, LateThr* thr) {
     const int lane = lane_id();
-            __shared__ float ths[kSplitMaxT + 1];
-            for (int t = threadIdx.x; t <= kSplitMaxT; t += 256) {
-                const float th = theta && t < T ? theta[t] : 0.0f;
-                ths[t] = (t < T && t >= t_min && th >= 1e-5f) ? th : __builtin_nanf("");
-                if (t < kSplitMaxT) thr->th[t] = ths[t];
+    __shared__ float ths[kSplitMaxT + 1];
+    for (int t = threadIdx.x; t <= kSplitMaxT; t += 256) {
+        const float th = theta && t < T ? theta[t] : 0.0f;
+        ths[t] = (t < T && t >= t_min && th >= 1e-5f) ? th : __builtin_nanf("");
+        if (t < kSplitMaxT) thr->th[t] = ths[t];
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        int lo = kSplitMaxT, hi = 0;
+#pragma unroll
+        for (int k = 0; k < kSplitMaxT / 64; ++k) {
+            const float x = ths[64 * k + lane];
+            const uint64_t v = __ballot(x == x);
+            if (v != 0) {
+                const int f = 64 * k + __ffsll((unsigned long long)v) - 1;
+                lo = f < lo ? f : lo;
+                hi = 64 * k + 64 - __clzll((long long)v);
             }
-            __syncthreads();
-            if (threadIdx.x < 64) {
-                int lo = kSplitMaxT, hi = 0;
-    #pragma unroll
-                for (int k = 0; k < kSplitMaxT / 64; ++k) {
-                    const float x = ths[64 * k + lane];
-                    const uint64_t v = __ballot(x == x);
-                    if (v != 0) {
-                        const int f = 64 * k + __ffsll((unsigned long long)v) - 1;
-                        lo = f < lo ? f : lo;
-                        hi = 64 * k + 64 - __clzll((long long)v);
-                    }
-                }
-                lo = lo < hi ? lo : hi;
-                // every step within [lo, hi) down or level (a NaN inside fails)
-                bool down = true;
-    #pragma unroll
-                for (int k = 0; k < kSplitMaxT / 64; ++k) {
-                    const int t = 64 * k + lane;
-                    if (t >= lo && t < hi - 1) down = down && ths[t] >= ths[t + 1];
-                }
-                const bool mono = __ballot(!down) == 0;
-                if (lane == 0) {
-                    const float l0 = hi > lo ? log2f(ths[lo]) : 0.0f, l1 = hi > lo ? log2f(ths[hi - 1]) : 0.0f;
-                    thr->lg0 = l0;
-                    thr->inv = l0 > l1 ? (float)(hi - 1 - lo) / (l0 - l1) : 0.0f;
-                    thr->lo = lo;
-                    thr->hi = hi;
-                    thr->mono = mono;
-                }
-            }
+        }
+        lo = lo < hi ? lo : hi;
+        // every step within [lo, hi) down or level (a NaN inside fails)
+        bool down = true;
+#pragma unroll
+        for (int k = 0; k < kSplitMaxT / 64; ++k) {
+            const int t = 64 * k + lane;
+            if (t >= lo && t < hi - 1) down = down && ths[t] >= ths[t + 1];
+        }
+        const bool mono = __ballot(!down) == 0;
+        if (lane == 0) {
+            const float l0 = hi > lo ? log2f(ths[lo]) : 0.0f, l1 = hi > lo ? log2f(ths[hi - 1]) : 0.0f;
+            thr->lg0 = l0;
+            thr->inv = l0 > l1 ? (float)(hi - 1 - lo) / (l0 - l1) : 0.0f;
+            thr->lo = lo;
+            thr->hi = hi;
+            thr->mono = mono;
+        }
+    }
 }
 
 struct SplitArgs {
@@ -1290,13 +1291,8 @@ int launch_integrate_split(vdttfs_ctx* ctx, float* out, const float* in, const f
     const int Cp = mf == 16 ? ceil16(s.C_in) : (s.C_in + 7) & ~7;
     unsigned char* sp = static_cast<unsigned char*>(scratch);
     float* a0 = reinterpret_cast<float*>(sp);
-    sp += align256((size_t)cols * ceil16(s.C_in) * 4);
     LateScratch sc;
-    sc.late = reinterpret_cast<int2*>(sp);
-    sp += align256((size_t)cols * s.C_in * 8);
-    sc.cnt = reinterpret_cast<int32_t*>(sp);
-    sp += align256((size_t)cols * 4);
-    sc.thr = reinterpret_cast<LateThr*>(sp);
+    carve(sp + align256((size_t)cols * ceil16(s.C_in) * 4), cols, s.C_in, &sc);
     VD_TRY(launch_split(ctx, SplitArgs{in, a0, sc.late, sc.cnt, alpha, theta, sc.thr, cols, s.C_in, Cp, ctx->c.T,
                                        ctx->c.alpha_by_time, t_min, mf == 16 ? 2 : 1, ctx->c.tfs}));
 

@@ -2,7 +2,9 @@
 // denominator (T1S = task1_lenet_mnist/stepbystep_cuda/snn_mnist_stepbystep.cu,
 // T2S = task2_vgg16_cifar10/stepbystep_cuda/bench_vgg_timedriven_baseline.cu):
 // every neuron takes every step of its windows, scans its whole receptive
-// field (no event lists), and fires once on the decaying threshold.
+// field (no event lists), and fires once on the decaying threshold.  The
+// programs scan the field at every step; k_step_layer scans it once for all of
+// them, so its time is no measure of theirs.
 //   k_step_layer  conv / FC layer, all its steps (T1S:47-103, T2S:53-108 and
 //                 141-200);
 //   k_step_pool   spiking 2x2 pool (T1S:107-127, T2S:110-139);
