@@ -168,6 +168,32 @@ def test_capture_without_scratch_is_refused_whole(gpu_ctx_factory):
     g.close()
 
 
+@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[3]], ids=lambda s: s[0])
+def test_counting_call_finds_its_scratch(gpu_ctx_factory, shape):
+    """A layer's first call also sizes what its counting call takes (merged
+    lists of 50 MB and more here): the counting call allocates nothing."""
+    print(f"scratch counting {shape[0]}", flush=True)
+    shape = shape[:5] + (96, 12, 12) + shape[8:]
+    name, T, tfs, task2, is_fc, B, H, W, C_in, C_out, K = shape
+    tc, ho, wo, Wt, bias, sp = case(shape, "random")
+    ctx = gpu_ctx_factory(tc)
+    alpha, theta = vdttfs.build_luts_host(tc, 0.75 * T, 0.5, 1.5 * T, 2.5)
+    d = [ctx.to_device(v) for v in (sp, Wt, bias, alpha, theta)]
+    out, again = ctx.empty(B * ho * wo * C_out), ctx.empty(B * ho * wo * C_out)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def free_bytes():
+        ctx.synchronize()
+        assert hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    ctx.layer_forward(out, *d, 3, B, H, W, C_in, ho, wo, C_out, K, K, False)
+    before = free_bytes()
+    eproc, _ = ctx.layer_forward(again, *d, 3, B, H, W, C_in, ho, wo, C_out, K, K, False, count=True)
+    assert eproc > 0 and before - free_bytes() < 16 << 20  # a kernel's first launch may load its code
+    np.testing.assert_array_equal(again.download(), out.download())
+
+
 def test_network_sizes_lists_for_the_layers_that_use_them(gpu_ctx_factory):
     """An FC layer at T = 64 never takes the split kernels, whose scratch would
     be half as large again as its merged lists (402 against 269 MB)."""

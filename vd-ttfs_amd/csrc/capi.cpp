@@ -68,6 +68,7 @@ int ensure_ref_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols) {
         if (ctx->ref_tin) VD_HIP(hipFree(ctx->ref_tin));
         if (ctx->ref_off) VD_HIP(hipFree(ctx->ref_off));
         ctx->ref_cin = ctx->ref_tin = ctx->ref_off = nullptr;
+        ctx->ref_elems = ctx->ref_cols = 0;
         VD_TRY(grow(&ctx->ref_cin, &h1, e * 4));
         VD_TRY(grow(&ctx->ref_tin, &h2, e * 4));
         VD_TRY(grow(&ctx->ref_off, &h3, c * (size_t)ctx->OS * 4));
@@ -86,6 +87,7 @@ int ensure_bin_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols) {
         if (ctx->bin_ev) VD_HIP(hipFree(ctx->bin_ev));
         if (ctx->bin_off) VD_HIP(hipFree(ctx->bin_off));
         ctx->bin_ev = ctx->bin_off = nullptr;
+        ctx->bin_elems = ctx->bin_cols = 0;
         VD_TRY(grow(&ctx->bin_ev, &h1, e * sizeof(vd_event)));
         VD_TRY(grow(&ctx->bin_off, &h2, c * (size_t)(ctx->c.T + 1) * 4));
         ctx->bin_elems = e;
@@ -404,19 +406,32 @@ static int engine_layer(vdttfs_ctx* ctx, float* d_out, const float* d_in, const 
     const bool lds_list = plan_lds_list(ctx, s, p, counters != nullptr, false);
     if (p.split == kSplitPixel && !counters)
         return launch_conv_px(ctx, d_out, d_in, d_lut_decay, d_kernel, d_bias, d_lut_th, t_min, s);
-    if (p.split && !counters && ensure_split_scratch(ctx, split_scratch_bytes(s)))
+    auto named_scratch = [&]() -> int {
+        if (!lds_list)
+            VD_TRY(ensure_merge_scratch(ctx, (size_t)(n_pix * cap), (size_t)n_pix * (ctx->c.T + 1)));
+        if (!dense) VD_TRY(ensure_bin_scratch(ctx, (size_t)cols * s.C_in, (size_t)cols));
+        return VDTTFS_OK;
+    };
+    if (p.split && !counters && ensure_split_scratch(ctx, split_scratch_bytes(s))) {
+        // A first call also sizes what the named plan would take, so that a
+        // counting call of the layer after it, or one captured when the split
+        // scratch no longer suffices, allocates nothing.  Where that much
+        // memory is not there, split calls ask no more.
+        if (!ctx->named_skip && named_scratch() == VDTTFS_E_NOMEM) {
+            ctx->named_skip = true;
+            (void)hipGetLastError();
+        }
         return p.split == kSplitLists
                    ? launch_integrate_lists(ctx, d_out, d_in, d_lut_decay, ctx->split_buf, d_kernel, d_bias,
                                             d_lut_th, t_min, s, nullptr)
                    : launch_integrate_split(ctx, d_out, d_in, d_lut_decay, ctx->split_buf, d_kernel, d_bias,
                                             d_lut_th, t_min, s);
-    if (!lds_list)
-        VD_TRY(ensure_merge_scratch(ctx, (size_t)(n_pix * cap), (size_t)n_pix * (ctx->c.T + 1)));
+    }
+    VD_TRY(named_scratch());
     if (dense)  // conv: merged lists straight from the dense map
         return launch_integrate_dense(ctx, d_out, d_in, d_lut_decay, (int2*)ctx->mrg_list, cap,
                                       (int32_t*)ctx->mrg_bstart, d_kernel, d_bias, d_lut_th, t_min, s,
                                       counters, nullptr, &p);
-    VD_TRY(ensure_bin_scratch(ctx, (size_t)cols * s.C_in, (size_t)cols));
     VD_TRY(launch_bucketize_bins(ctx, d_in, cols, s.C_in, d_lut_decay, (vd_event*)ctx->bin_ev,
                                  (int32_t*)ctx->bin_off, nullptr));
     return launch_integrate_bins(ctx, d_out, (const vd_event*)ctx->bin_ev, (const int32_t*)ctx->bin_off,

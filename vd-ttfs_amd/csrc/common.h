@@ -42,6 +42,7 @@ struct vdttfs_ctx {
     size_t split_bytes;
     bool split_captured;
     std::vector<void*> split_kept;
+    bool named_skip;  // a split call could not size its named plan's scratch too
     unsigned long long* d_counters;  // kCounterStripes x 4 u64 (summed on the host)
     hipEvent_t timer[2];             // vdttfs_timer_begin/end (created on first use)
     bool timer_ready;
