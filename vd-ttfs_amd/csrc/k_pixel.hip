@@ -28,6 +28,9 @@ namespace {
 constexpr int kPxMaxEl = 160;  // a key holds an element in 8 bits
 constexpr int kPxMaxOut = 16;
 
+// N: elements that the tables hold, 32 or kPxMaxEl (a launch of a few
+// microseconds feels a kilobyte of arguments).
+template <int N>
 struct PxArgs {
     const float* in;     // [n_cols][C_in] spike times (NHWC map)
     const float* alpha;  // decay LUT, T + 1 entries
@@ -43,7 +46,7 @@ struct PxArgs {
     FastDiv div_w, div_h;
     // element e: its offset from the field's first element, and its tap's row
     // << 16 | column
-    int dk[kPxMaxEl], tap[kPxMaxEl];
+    int dk[N], tap[N];
 };
 
 // The smallest value of a group of G lanes.
@@ -57,7 +60,7 @@ __device__ __forceinline__ unsigned group_min(unsigned v) {
 
 // G lanes share a pixel: each holds CO outputs and NEL elements, e = G i + g.
 template <int G, int CO, int NEL>
-__global__ __launch_bounds__(256) void k_conv_px(PxArgs a) {
+__global__ __launch_bounds__(256) void k_conv_px(PxArgs<(G > 1 ? kPxMaxEl : 32)> a) {
     constexpr int COP = G * ((CO + 3) & ~3);
     constexpr unsigned kNone = ~0u;
     __shared__ __attribute__((aligned(16))) float w_lds[G * NEL * COP];
@@ -265,10 +268,12 @@ bool conv_px_ok(int T, const IntegShape& s) {
     return T > 64 || s.C_out <= 8 || nel <= 16 || pix >= 12288;
 }
 
-int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W, const float* bias,
-                   const float* theta, int t_min, const IntegShape& s) {
-    if (!conv_px_ok(ctx->c.T, s) || ctx->c.T > 255) return set_error(VDTTFS_E_UNSUPPORTED, "conv_px: layer outside its limits");
-    PxArgs a{};
+namespace {
+
+template <int N>
+PxArgs<N> px_args(const vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W,
+                  const float* bias, const float* theta, int t_min, const IntegShape& s) {
+    PxArgs<N> a{};
     a.in = in;
     a.alpha = alpha;
     a.W = W;
@@ -276,7 +281,6 @@ int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* al
     a.theta = theta;
     a.out = out;
     a.n_pix = s.B * s.H_out * s.W_out;
-    if (a.n_pix <= 0) return VDTTFS_OK;
     a.T = ctx->c.T;
     a.t_min = t_min;
     a.alpha_by_time = ctx->c.alpha_by_time;
@@ -289,7 +293,7 @@ int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* al
     a.C_out = s.C_out;
     a.pad_h = s.pad_h;
     a.pad_w = s.pad_w;
-    a.nel = s.K_h * s.K_w * s.C_in;
+    a.nel = s.K_h * s.K_w * s.C_in;  // at most N
     a.in_bytes = s.B * s.H_in * s.W_in * s.C_in * 4;
     a.inside = s.pad_h == 0 && s.pad_w == 0 && s.H_out <= s.H_in - s.K_h + 1 && s.W_out <= s.W_in - s.K_w + 1;
     a.div_w = make_fastdiv(s.W_out);
@@ -300,36 +304,48 @@ int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* al
                 a.dk[e] = (kh * s.W_in + kw) * s.C_in + ci;
                 a.tap[e] = kh << 16 | kw;
             }
+    return a;
+}
+
+}  // namespace
+
+int launch_conv_px(vdttfs_ctx* ctx, float* out, const float* in, const float* alpha, const float* W, const float* bias,
+                   const float* theta, int t_min, const IntegShape& s) {
+    if (!conv_px_ok(ctx->c.T, s) || ctx->c.T > 255) return set_error(VDTTFS_E_UNSUPPORTED, "conv_px: layer outside its limits");
+    const int n_pix = s.B * s.H_out * s.W_out, nel = s.K_h * s.K_w * s.C_in;
+    if (n_pix <= 0) return VDTTFS_OK;
     // few pixels: one wave per workgroup, so that they spread over the CUs
-    const int threads = a.n_pix >= 256 * 256 ? 256 : 64;
-    const int G = a.nel > 32 ? 4 : 1;
-    const dim3 grid((unsigned)(((int64_t)a.n_pix * G + threads - 1) / threads)), block(threads);
-#define VD_PX(G_, C, N) hipLaunchKernelGGL((k_conv_px<G_, C, N>), grid, block, 0, ctx->stream, a)
+    const int threads = n_pix >= 256 * 256 ? 256 : 64;
+    const int G = nel > 32 ? 4 : 1;
+    const dim3 grid((unsigned)(((int64_t)n_pix * G + threads - 1) / threads)), block(threads);
+#define VD_PX(G_, C, N)                                                              \
+    hipLaunchKernelGGL((k_conv_px<G_, C, N>), grid, block, 0, ctx->stream,           \
+                       px_args<(G_ > 1 ? kPxMaxEl : 32)>(ctx, out, in, alpha, W, bias, theta, t_min, s))
 #define VD_PX_N(C)            \
     do {                      \
-        if (a.nel <= 9)       \
+        if (nel <= 9)         \
             VD_PX(1, C, 9);   \
-        else if (a.nel <= 16) \
+        else if (nel <= 16)   \
             VD_PX(1, C, 16);  \
-        else if (a.nel <= 25) \
+        else if (nel <= 25)   \
             VD_PX(1, C, 25);  \
         else                  \
             VD_PX(1, C, 32);  \
     } while (0)
     if (G > 1) {
-        if (a.nel <= 64)
+        if (nel <= 64)
             VD_PX(4, 4, 16);
-        else if (a.nel <= 112)
+        else if (nel <= 112)
             VD_PX(4, 4, 28);
         else
             VD_PX(4, 4, 40);
-    } else if (a.C_out <= 4)
+    } else if (s.C_out <= 4)
         VD_PX_N(4);
-    else if (a.C_out <= 6)
+    else if (s.C_out <= 6)
         VD_PX_N(6);
-    else if (a.C_out <= 8)
+    else if (s.C_out <= 8)
         VD_PX_N(8);
-    else if (a.C_out <= 12)
+    else if (s.C_out <= 12)
         VD_PX_N(12);
     else
         VD_PX_N(16);
