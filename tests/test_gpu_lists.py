@@ -34,14 +34,19 @@ SHAPES = [
 ]
 # either side of the lengths up to which a layer takes the lists
 LENGTHS = [
-    ("t80-fc-2048-70", 80, 0, True, True, 31, 1, 1, 2048, 70, 1),
-    ("t80-fc-2049-70", 80, 0, True, True, 31, 1, 1, 2049, 70, 1),
     ("t80-fc-4096-70", 80, 0, True, True, 33, 1, 1, 4096, 70, 1),
     ("t80-fc-4097-70", 80, 0, True, True, 33, 1, 1, 4097, 70, 1),
+    ("t80-fc-8192-140", 80, 0, True, True, 4, 1, 1, 8192, 140, 1),
+    ("t80-fc-8193-140", 80, 0, True, True, 4, 1, 1, 8193, 140, 1),
+    ("t80-fc-8192-132-b65", 80, 0, True, True, 65, 1, 1, 8192, 132, 1),
     ("t80-conv3-256-140", 80, 0, True, False, 2, 5, 4, 256, 140, 3),
     ("t80-conv3-257-140", 80, 0, True, False, 2, 5, 4, 257, 140, 3),
-    ("t80-conv5-80-20", 80, 0, True, False, 1, 5, 4, 80, 20, 5),
-    ("t80-conv5-81-20", 80, 0, True, False, 1, 5, 4, 81, 20, 5),
+    ("t80-conv3-455-20", 80, 0, True, False, 1, 5, 4, 455, 20, 3),
+    ("t80-conv3-456-20", 80, 0, True, False, 1, 5, 4, 456, 20, 3),
+    ("t80-conv5-128-20", 80, 0, True, False, 1, 5, 4, 128, 20, 5),
+    ("t80-conv5-129-20", 80, 0, True, False, 1, 5, 4, 129, 20, 5),
+    ("t80-conv5-200-140", 80, 0, True, False, 1, 5, 4, 200, 140, 5),
+    ("t80-conv5-201-140", 80, 0, True, False, 1, 5, 4, 201, 140, 5),
 ]
 
 

@@ -128,7 +128,7 @@ def tile_of(shape):
     tiles = -(-pix // 32) * -(-C_out // 32)
     if C_out < 32 or 4 * tfs < T or T > 128:
         return None
-    if taps > 9 and nel > 3000:
+    if taps > 9 and nel > (6400 if C_out > 128 and pix <= 512 else 3750):
         return None
     if T > 64:
         if nel <= 300 or taps == 1 or (nel <= 576 and pix <= 1024):
@@ -160,9 +160,12 @@ LINES = [  # either side of the lines that the split is chosen by
     ((16, 16), ("t80-conv3-65-40", 80, 40, True, False, 3, 9, 7, 65, 40, 3)),
     (None, ("t80-conv1-601-40", 80, 40, True, False, 3, 9, 7, 601, 40, 1)),
     # long fields of many taps the merged lists
-    ((16, 16), ("t64-conv5-120-140", 64, 32, True, False, 2, 6, 5, 120, 140, 5)),
-    (None, ("t64-conv5-121-40", 64, 32, True, False, 2, 6, 5, 121, 40, 5)),
-    (None, ("t80-conv5-121-40", 80, 40, True, False, 2, 6, 5, 121, 40, 5)),
+    ((16, 16), ("t64-conv5-150-40", 64, 32, True, False, 2, 6, 5, 150, 40, 5)),
+    (None, ("t64-conv5-151-40", 64, 32, True, False, 2, 6, 5, 151, 40, 5)),
+    (None, ("t80-conv5-151-128", 80, 40, True, False, 2, 6, 5, 151, 128, 5)),
+    ((16, 16), ("t64-conv5-256-132", 64, 32, True, False, 2, 6, 5, 256, 132, 5)),
+    (None, ("t64-conv5-257-132", 64, 32, True, False, 2, 6, 5, 257, 132, 5)),
+    (None, ("t64-conv5-151-132-513", 64, 32, True, False, 9, 19, 3, 151, 132, 5)),
     (None, ("t64-conv3-15-99", 64, 32, True, False, 16, 32, 16, 15, 99, 3)),
     ((32, 32), ("t64-conv3-16-99", 64, 32, True, False, 16, 32, 16, 16, 99, 3)),
 ]

@@ -1016,11 +1016,11 @@ bool split_ok(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
     // not serve (T > 64, or more than 9 taps: bucketize or dense merge and a
     // stream) that is any layer of a few inputs past nine taps, until the list
     // comes in many windows, each of which reads it from its start (times as
-    // fast as merged lists at densities 0.1 / 0.3 / 0.7: 64 outputs, 64 pixels,
-    // 2,500 elements 1.21 / 1.34 / 1.15, 3,500 1.13 / 1.27 / 0.90, 5,000 1.02 /
-    // 0.98 / 0.72; 200 outputs, 4,096 pixels, 2,500 0.87 / 1.14 / 1.33, 5,000
-    // 0.72 / 1.03 / 1.25).
-    if (taps > 9 && K > 3000) return false;
+    // fast as merged lists at densities 0.1 / 0.3 / 0.7, T = 80: 64 outputs, 64
+    // pixels, 2,750 elements 1.36 / 1.45 / 1.28, 3,750 1.08 / 1.08 / 0.93, 6,400
+    // 0.93 / 0.98 / 0.61; two waves a list: 200 outputs, 512 pixels, 6,400 1.31 /
+    // 1.56 / 1.48, but 4,096 pixels 5,000 0.89 / 1.13 and 3,750 1.00 / 1.19 / 1.34).
+    if (taps > 9 && K > (s.C_out > 128 && pix <= 512 ? 6400 : 3750)) return false;
     if (T <= 64 && taps > 9) return K >= 4;
     // Past 64 steps the lists of every bin (two launches) are there as well and
     // finish first in short fields, where the split even lost to the kernels
@@ -1099,18 +1099,21 @@ bool lists_fit(const vdttfs_ctx* ctx, const IntegShape& s) {
 //
 // So do long lists: one past `cap` entries is read from its start for every
 // window of it, where the merged lists are read once.  Times as fast as those,
-// T = 80: FC to 128 outputs, 32 images, densities 0.05 / 0.3 / 1: 2,000 inputs
-// 1.34 / 1.47 / 1.16, 4,096 1.13 / 1.21 / 0.77, 8,192 1.01 / 0.91 / 0.67, 16,384
-// 0.83 / 0.86 / 0.42; one image to 10 outputs 2,000 1.37 / 1.10 / 0.88, 4,096
-// 1.03 / 0.92 / 0.58; 3x3, 512 channels, 1,024 pixels, densities 0.1 / 0.7: 128
-// outputs 1.84 / 1.11, 512 outputs 1.20 / 0.65; 5x5, 200 channels (each entry's
-// tap is found among 25): 32 outputs 1.65 / 0.34, 128 1.64 / 0.50.
+// T = 80: FC to 64 outputs, 30 images, densities 0.05 / 0.2 / 0.5: 2,500 inputs
+// 1.32 / 1.42 / 1.39, 4,096 1.17 / 1.35 / 0.97; one image to 10 outputs 2,500 1.23 /
+// 1.15 / 0.97, 4,096 1.04 / 0.98 / 0.77; 128 outputs, 32 images, densities 0.05 /
+// 0.3 / 1: 8,192 1.01 / 0.91 / 0.67, 16,384 0.83 / 0.86 / 0.42; 1,000 outputs, 32
+// images, 8,192 0.96 / 1.45 / 1.34, 256 images 0.81 at 0.05.  3x3, 512 channels,
+// 1,024 pixels, densities 0.1 / 0.7: 128 outputs 1.84 / 1.11, 512 outputs 1.20 /
+// 0.65.  5x5 (each entry's tap is found among 25), 512 pixels, densities 0.1 / 0.3 /
+// 0.7: 64 outputs 2,750 elements 2.41 / 1.42 / 0.71, 3,750 2.15 / 1.08 / 0.48; 200
+// outputs 3,750 2.53 / 1.68 / 0.93, 5,000 2.42 / 1.43 / 0.80, 6,400 2.00 / 1.18 / 0.68.
 bool lists_ok(const vdttfs_ctx* ctx, const IntegShape& s) {
     if (ctx->c.T <= 64 || !lists_fit(ctx, s)) return false;
     const int taps = s.is_fc ? 1 : s.K_h * s.K_w, K = taps * s.C_in;
-    if (taps > 9) return K <= 2000;
-    if (taps > 1 && s.C_out > 128) return K <= 2304;
-    return K <= (split_pix(s) < 32 ? 2048 : 4096);
+    if (taps > 9) return K <= (s.C_out > 128 ? 5000 : 3200);
+    if (taps > 1) return K <= (s.C_out > 128 ? 2304 : 4096);
+    return K <= (s.C_out > 128 && split_pix(s) <= 64 ? 8192 : 4096);
 }
 
 int split_choice(const vdttfs_ctx* ctx, const IntegShape& s, bool net) {
