@@ -78,18 +78,24 @@ int ensure_ref_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols) {
     return VDTTFS_OK;
 }
 
+// Two buffers in one allocation (hipMalloc is what a first call waits for):
+// *first of n1 bytes, *second of n2 behind it.
+static int grow_pair(void** first, size_t n1, void** second, size_t n2) {
+    const size_t at = (n1 + 255) & ~size_t(255);
+    size_t have = 0;
+    *second = nullptr;
+    VD_TRY(grow(first, &have, at + n2));
+    *second = static_cast<unsigned char*>(*first) + at;
+    return VDTTFS_OK;
+}
+
 int ensure_bin_scratch(vdttfs_ctx* ctx, size_t elems, size_t cols) {
     if (elems > ctx->bin_elems || cols > ctx->bin_cols || !ctx->bin_ev) {
         VD_TRY(before_growth(ctx));
-        size_t e = elems > ctx->bin_elems ? elems : ctx->bin_elems;
-        size_t c = cols > ctx->bin_cols ? cols : ctx->bin_cols;
-        size_t h1 = 0, h2 = 0;
-        if (ctx->bin_ev) VD_HIP(hipFree(ctx->bin_ev));
-        if (ctx->bin_off) VD_HIP(hipFree(ctx->bin_off));
-        ctx->bin_ev = ctx->bin_off = nullptr;
+        const size_t e = elems > ctx->bin_elems ? elems : ctx->bin_elems;
+        const size_t c = cols > ctx->bin_cols ? cols : ctx->bin_cols;
         ctx->bin_elems = ctx->bin_cols = 0;
-        VD_TRY(grow(&ctx->bin_ev, &h1, e * sizeof(vd_event)));
-        VD_TRY(grow(&ctx->bin_off, &h2, c * (size_t)(ctx->c.T + 1) * 4));
+        VD_TRY(grow_pair(&ctx->bin_ev, e * sizeof(vd_event), &ctx->bin_off, c * (size_t)(ctx->c.T + 1) * 4));
         ctx->bin_elems = e;
         ctx->bin_cols = c;
     }
@@ -114,15 +120,10 @@ int read_counters(vdttfs_ctx* ctx, unsigned long long out[4]) {
 int ensure_merge_scratch(vdttfs_ctx* ctx, size_t list_elems, size_t bstart_elems) {
     if (list_elems > ctx->mrg_list_elems || bstart_elems > ctx->mrg_bstart_elems || !ctx->mrg_list) {
         VD_TRY(before_growth(ctx));
-        size_t e = list_elems > ctx->mrg_list_elems ? list_elems : ctx->mrg_list_elems;
-        size_t b = bstart_elems > ctx->mrg_bstart_elems ? bstart_elems : ctx->mrg_bstart_elems;
-        size_t h1 = 0, h2 = 0;
-        if (ctx->mrg_list) VD_HIP(hipFree(ctx->mrg_list));
-        if (ctx->mrg_bstart) VD_HIP(hipFree(ctx->mrg_bstart));
-        ctx->mrg_list = ctx->mrg_bstart = nullptr;
+        const size_t e = list_elems > ctx->mrg_list_elems ? list_elems : ctx->mrg_list_elems;
+        const size_t b = bstart_elems > ctx->mrg_bstart_elems ? bstart_elems : ctx->mrg_bstart_elems;
         ctx->mrg_list_elems = ctx->mrg_bstart_elems = 0;
-        VD_TRY(grow(&ctx->mrg_list, &h1, e * sizeof(int2)));
-        VD_TRY(grow(&ctx->mrg_bstart, &h2, b * 4));
+        VD_TRY(grow_pair(&ctx->mrg_list, e * sizeof(int2), &ctx->mrg_bstart, b * 4));
         ctx->mrg_list_elems = e;
         ctx->mrg_bstart_elems = b;
     }
@@ -226,8 +227,8 @@ int vdttfs_destroy(vdttfs_ctx* ctx) {
     if (!ctx) return VDTTFS_OK;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    void* bufs[] = {ctx->ref_cin, ctx->ref_tin,    ctx->ref_off,   ctx->bin_ev,
-                    ctx->bin_off, ctx->mrg_list, ctx->mrg_bstart, ctx->d_counters, ctx->split_buf};
+    void* bufs[] = {ctx->ref_cin,  ctx->ref_tin,     ctx->ref_off,  ctx->bin_ev,
+                    ctx->mrg_list, ctx->d_counters, ctx->split_buf};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (void* b : ctx->split_kept) (void)hipFree(b);

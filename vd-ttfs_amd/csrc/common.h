@@ -30,11 +30,11 @@ struct vdttfs_ctx {
     size_t ref_elems, ref_cols;
     // engine bin-layout scratch
     void* bin_ev;
-    void* bin_off;
+    void* bin_off;  // in bin_ev's allocation
     size_t bin_elems, bin_cols;
     // engine merged per-pixel event lists
     void* mrg_list;
-    void* mrg_bstart;
+    void* mrg_bstart;  // in mrg_list's allocation
     size_t mrg_list_elems, mrg_bstart_elems;
     // scratch of the split and list kernels.  split_captured: a captured graph
     // holds its address, so growth sets it aside until the context ends
